@@ -66,8 +66,9 @@ typedef struct {
 } CtGemm;
 
 void ctk_gemm(const CtGemm *g, hipStream_t s);
-/* Tests: 128 or 256 forces the pre-split kernels' tile (0: the tile-count
- * model); sizeof(CtGemm) for the tests' struct mirror. */
+/* Tests: 128 or 256 forces the pre-split kernels' tile, rows * 1000 + columns
+ * a few-row tile (16016, 16032, 32032, 32064, 64128; 0: the cost model);
+ * sizeof(CtGemm) for the tests' struct mirror. */
 void ctk_gemm_force_tile(int rows);
 int  ctk_gemm_sizeof(void);
 

@@ -14,8 +14,10 @@
 // fmadd), 300-311 (GLU), 398-408 / 466-476 (KV-cache row scatter).
 #include "ct_dev.h"
 #include "ct_launch.h"
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
+#include <utility>
 
 namespace {
 
@@ -1356,6 +1358,388 @@ __global__ __launch_bounds__(512) void gemm_split256_sp_kernel(CtGemm g, int n_m
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few-row encoder GEMM: small tiles, so that the rows of one clip or a few
+// (13 to about 2000) fill the chip.  With the 128-row tiles a 1280-column
+// product of an 8 s clip (101 rows) ran on 5 or 10 CUs and took the time of
+// one tile's K loop.  A row's K loop stays one chain of MFMAs in the same
+// order (K-steps, hi then lo), so the bits are those of the other kernels;
+// K is not split.
+//
+// What bounds it is the instruction issue of single wavefronts (one
+// instruction per about 7 cycles when a SIMD holds one wave), then the DMA's
+// L2 traffic.  So the roles are separated: WR x WC waves run nothing but
+// fragment reads (a stage ahead, into a second register set) and MFMAs; the
+// waves from P0 on fetch the stages (KS of K, a ring of NS) by LDS DMA at a
+// scalar base and a constant lane offset, and, for fp32 activations, split
+// each 16 x 32 fragment into hi and lo once per workgroup, two stages ahead.
+// One barrier per stage.  LDS rows are swizzled for both the DMA (1 KB runs)
+// and the fragment reads.  In the 64 x 128 tile every wave does both.
+//
+// Measured (us; before -> now): fp32 activations 13 x 1280 x 1280 15 -> 6.6,
+// 101 x 1280 x 5120 161 -> 21, 376 x 5120 x 1280 49 -> 22; hi + lo planes
+// 101 x 1280 x 5120 114 -> 13, 1008 x 1280 x 5120 115 -> 46; hi alone
+// 101 x 1280 x 5120 76 -> 10 (13 MB of weights).
+// ---------------------------------------------------------------------------
+enum { A_F32 = 0, A_HILO = 1, A_HI = 2 };
+
+template <int AM_, int RB_, int CB_, int WR_, int WC_, int P0_, int NW_, int KS_, int NS_>
+struct RowsCfg {
+    static constexpr int AM = AM_, RB = RB_, CB = CB_, WR = WR_, WC = WC_, P0 = P0_, NW = NW_, KS = KS_, NS = NS_;
+    static constexpr int TM = 16 * RB * WR, TN = 16 * CB * WC;
+    static constexpr int A_BYTES = TM * KS * (AM == A_HI ? 2 : 4), W_BYTES = TN * KS * 2;
+    static constexpr int STAGE = A_BYTES + W_BYTES;           // A fp32 | A hi, A lo | A hi, then W
+    static constexpr int KN = KS / 32, NF = AM == A_F32 ? TM / 16 * KN : 0;   // fragments split per stage
+    static constexpr int NI_A = A_BYTES / 1024, NI = STAGE / 1024;
+    static constexpr int P = NW - P0, PW = NI / P;            // producer waves, DMA instructions of each per stage
+    static constexpr int AHEAD = AM == A_F32 ? 2 : 1;
+    static constexpr int LDS = NS * STAGE + 2 * NF * 2048;
+    static constexpr int PL = AM == A_HILO ? NI_A / 2 : NI_A; // DMA instructions per A plane
+    static_assert(NI % P == 0 && PL % P == 0, "each DMA instruction j is of one operand for every producer");
+    static_assert((NS - 1) * PW <= 63, "vmcnt counts to 63");
+    static_assert(LDS <= 160 * 1024 && WR * WC <= NW && NS > AHEAD, "LDS and wave budget");
+};
+
+// One 16-byte-per-lane DMA as lds_dma16_asm, from base + off to LDS byte
+// lds + IMM: the address is a scalar base and a 32-bit lane offset, so a step
+// along K costs no vector instruction.
+template <int IMM>
+__device__ __forceinline__ void lds_dma16_saddr(const char *base, unsigned off, unsigned lds) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds),
+                 "i"(IMM) : "memory", "scc");
+}
+
+// 16-byte slot of chunk c in LDS row R of NCH chunks.  Rows of 16 chunks or
+// more start on the same bank, so 16 rows take 16 slots; rows of 8 chunks
+// alternate between two halves of the banks.
+template <int NCH>
+__device__ __forceinline__ int rswz(int R, int c) {
+    return c ^ (NCH >= 16 ? (R & 15) : ((R & 7) ^ ((R >> 3) & 1)));
+}
+
+// split_bf16 of eight values, two per conversion instruction
+__device__ __forceinline__ void split8(float4 x0, float4 x1, bf16x8 &hi, bf16x8 &lo) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x[2 * i], x[2 * i + 1]}, bf16x2));
+        const float r0 = x[2 * i] - __uint_as_float(h[i] << 16), r1 = x[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u);
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){r0, r1}, bf16x2));
+    }
+    hi = __builtin_bit_cast(bf16x8, h);
+    lo = __builtin_bit_cast(bf16x8, l);
+}
+
+// s_waitcnt vmcnt(y * PW) lgkmcnt(0) for a runtime y <= Y
+template <int Y, int PW>
+__device__ __forceinline__ void wait_younger(int y) {
+    if constexpr (Y > 0) {
+        if (y < Y) {
+            wait_younger<Y - 1, PW>(y);
+            return;
+        }
+    }
+    constexpr int v = Y * PW;
+    __builtin_amdgcn_s_waitcnt((v & 15) | (7 << 4) | ((v >> 4) << 14));
+}
+
+template <class C, int... J>
+__device__ __forceinline__ void dma_stage(const char *pA, const char *pL, const char *pW, const unsigned (&off)[C::PW],
+                                          unsigned lds, std::integer_sequence<int, J...>) {
+    (lds_dma16_saddr<C::P * J * 1024>(C::P * J >= C::NI_A ? pW : C::P * J >= C::PL ? pL : pA, off[J], lds), ...);
+}
+
+template <class C, bool GLU>
+__device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char *smem) {
+    constexpr int AM = C::AM, RB = C::RB, CB = C::CB, KS = C::KS, NS = C::NS, PW = C::PW, P = C::P, KN = C::KN;
+    constexpr int EA = AM == A_F32 ? 4 : 2;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    const int tm = t % n_mt, tn = t / n_mt;
+    const int m0 = tm * C::TM;
+    constexpr int CO = GLU ? CB / 2 : CB;                 // output column blocks of a wave
+    const int c0 = tn * 16 * CO * C::WC;                  // first output column
+    const int nlim = GLU ? 2 * g.glu_half : g.N;
+    // weight row of tile row R (GLU: each wave's group holds its value
+    // columns, then their gates)
+    auto wcol = [&](int R) {
+        if (!GLU) return c0 + R;
+        const int grp = R / (16 * CB), q = R % (16 * CB);
+        return q < 16 * CO ? c0 + grp * 16 * CO + q : g.glu_half + c0 + grp * 16 * CO + q - 16 * CO;
+    };
+    const bool comp = wv < C::WR * C::WC, prod = wv >= C::P0;
+    const int pw = wv - C::P0;
+    // DMA instruction i = pw + P*j of a stage fills its LDS bytes [1024 i, 1024 i + 1024)
+    unsigned off[PW];
+#pragma unroll
+    for (int j = 0; j < PW; j++) {
+        const int i = pw + P * j;
+        if (P * j < C::NI_A) {
+            constexpr int NCH = KS * EA / 16, RPI = 64 / NCH;
+            const int R = (i % C::PL) * RPI + lane / NCH, ch = rswz<NCH>(R, lane % NCH);
+            off[j] = (unsigned)((min(m0 + R, g.M - 1) - m0) * (int)g.lda * EA + ch * 16);   // rows >= M are never stored
+        } else {
+            constexpr int NCH = KS / 8, RPI = 64 / NCH;
+            const int R = (i - C::NI_A) * RPI + lane / NCH, ch = rswz<NCH>(R, lane % NCH);
+            off[j] = (unsigned)((min(wcol(R), nlim - 1) - c0) * g.K * 2 + ch * 16);
+        }
+    }
+    // the next stage to fetch: its rows' start in each operand, its slot
+    const char *pA = (AM == A_F32 ? (const char *)g.A : (const char *)g.Ahi) + (long)m0 * g.lda * EA;
+    const char *pL = AM == A_HILO ? (const char *)(g.Alo + (long)m0 * g.lda) : nullptr;
+    const char *pW = (const char *)(g.W + (long)c0 * g.K);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr_t)smem) + pw * 1024;
+    int slot = 0;
+    auto issue = [&]() {
+        dma_stage<C>(pA, pL, pW, off, lds0 + slot, std::make_integer_sequence<int, PW>());
+        pA += KS * EA;
+        if (AM == A_HILO) pL += KS * EA;
+        pW += KS * 2;
+        slot = slot + C::STAGE == NS * C::STAGE ? 0 : slot + C::STAGE;
+    };
+    const int wr = wv / C::WC, wc = wv % C::WC;
+    // bias and the residual rows first (at clamped indices, used after the
+    // loop): their latency passes under the K loop
+    uint16_t bia[CB];
+    float yres[RB][CO][4];
+    const bool fm = !GLU && g.nseg == 0 && !g.row_len && g.epi == CT_EPI_FMADD;
+    const uint16_t *bp = g.bias ? g.bias : g.W;
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) bia[cb] = bp[min(wcol((wc * CB + cb) * 16 + r), nlim - 1)];
+    if (fm) {
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+            for (int cb = 0; cb < CO; cb++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j, col = c0 + (wc * CO + cb) * 16 + r;
+                    yres[rb][cb][j] = g.Y[(long)min(m, g.M - 1) * g.ldy + min(col, g.N - 1)];
+                }
+    } else {
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+            for (int cb = 0; cb < CO; cb++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) yres[rb][cb][j] = 0.0f;
+    }
+    f32x4 acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < CB; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // Fragments of one stage in registers; two sets, so that a stage's reads
+    // run under the MFMAs of the stage before.
+    struct Frag { u16x8 w[KN][CB], h[KN][RB], l[KN][AM == A_HI ? 1 : RB]; };
+    // per-lane LDS offsets within a stage (or a fragment buffer), per K-step
+    int offA[KN], offW[KN];
+#pragma unroll
+    for (int ks = 0; ks < KN; ks++) {
+        const int lo = r * KS * 2 + rswz<KS / 8>(r, ks * 4 + kg) * 16;
+        offA[ks] = AM == A_F32 ? NS * C::STAGE + (wr * RB * KN + ks) * 2048 + lane * 16 : wr * RB * 16 * KS * 2 + lo;
+        offW[ks] = C::A_BYTES + wc * CB * 16 * KS * 2 + lo;
+    }
+    int rslot = 0;           // slot of the next stage to read
+    auto read = [&](int par, Frag &f) {
+#pragma unroll
+        for (int ks = 0; ks < KN; ks++) {
+            const char *pa = smem + offA[ks] + (AM == A_F32 ? par * (C::NF * 2048) : rslot);
+            const char *pw_ = smem + offW[ks] + rslot;
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+                const char *p = pa + rb * (AM == A_F32 ? KN * 2048 : 16 * KS * 2);
+                f.h[ks][rb] = *reinterpret_cast<const u16x8 *>(p);
+                if constexpr (AM != A_HI)
+                    f.l[ks][rb] = *reinterpret_cast<const u16x8 *>(p + (AM == A_F32 ? 1024 : C::TM * KS * 2));
+            }
+#pragma unroll
+            for (int cb = 0; cb < CB; cb++) f.w[ks][cb] = *reinterpret_cast<const u16x8 *>(pw_ + cb * 16 * KS * 2);
+        }
+        rslot = rslot + C::STAGE == NS * C::STAGE ? 0 : rslot + C::STAGE;
+    };
+    // fp32 rows of a stage -> hi/lo fragments, once per workgroup: fragment f
+    // is row block f / KN, K-step f % KN, 2 KB (hi then lo, in lane order) of
+    // the parity's buffer
+    constexpr int QF = (C::NF + P - 1) / P;
+    int offX[QF + 1][2];
+#pragma unroll
+    for (int q = 0; q < QF; q++) {
+        const int f = min(pw + P * q, C::NF - 1), c = f % KN * 8 + kg * 2;
+        offX[q][0] = (f / KN * 16 + r) * KS * 4 + rswz<KS / 4>(r, c) * 16;
+        offX[q][1] = (f / KN * 16 + r) * KS * 4 + rswz<KS / 4>(r, c + 1) * 16;
+    }
+    int sslot = 0;           // slot of the next stage to split
+    auto split = [&](int par) {
+        char *fr = smem + NS * C::STAGE + pw * 2048 + lane * 16 + par * (C::NF * 2048);
+        float4 x[QF + 1][2];
+#pragma unroll
+        for (int q = 0; q < QF; q++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) x[q][e] = *reinterpret_cast<const float4 *>(smem + offX[q][e] + sslot);
+#pragma unroll
+        for (int q = 0; q < QF; q++) {
+            if (C::NF % P && pw + P * q >= C::NF) break;
+            bf16x8 hi, lo;
+            split8(x[q][0], x[q][1], hi, lo);
+            *reinterpret_cast<bf16x8 *>(fr + P * q * 2048) = hi;
+            *reinterpret_cast<bf16x8 *>(fr + P * q * 2048 + 1024) = lo;
+        }
+        sslot = sslot + C::STAGE == NS * C::STAGE ? 0 : sslot + C::STAGE;
+    };
+    auto mma = [&](const Frag &f) {
+#pragma unroll
+        for (int ks = 0; ks < KN; ks++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+#pragma unroll
+                for (int cb = 0; cb < CB; cb++)
+                    acc[rb][cb] = mfma16(as_bf16x8(f.h[ks][rb]), as_bf16x8(f.w[ks][cb]), acc[rb][cb]);
+                if constexpr (AM != A_HI) {
+#pragma unroll
+                    for (int cb = 0; cb < CB; cb++)
+                        acc[rb][cb] = mfma16(as_bf16x8(f.l[ks][rb]), as_bf16x8(f.w[ks][cb]), acc[rb][cb]);
+                }
+            }
+    };
+    const int nk = g.K / KS;
+    // all but this wave's y youngest stages of DMA landed and its LDS accesses
+    // done, for every wave
+    auto landed = [&](int y) {
+        wait_younger<NS - 1, PW>(y);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    asm volatile("" ::: "memory");
+    if (prod) {
+#pragma unroll
+        for (int p = 0; p < NS; p++)
+            if (p < nk) issue();
+    }
+    Frag f0, f1;
+    landed(min(nk, NS) - 1);
+    if constexpr (AM == A_F32) {
+        if (prod) split(0);
+        landed(max(0, min(nk, NS) - 2));
+        if (prod && nk > 1) split(1);
+    }
+    if (comp) read(0, f0);
+    // Step kt (its fragments in cur, par its parity): every wave is done with
+    // stage kt's slot, which is refilled; stage kt + 1's fragments are read,
+    // and (fp32) stage kt + 2 is split, while stage kt's MFMAs run.
+    int kt = 0;
+    auto step = [&](int par, const Frag &cur, Frag &nxt) {       // kt + NS < nk
+        constexpr int v = (NS - 1 - C::AHEAD) * PW;
+        __builtin_amdgcn_s_waitcnt((v & 15) | (7 << 4) | ((v >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (comp) read(par ^ 1, nxt);
+        if (prod) {
+            issue();
+            if (AM == A_F32) split(par);
+        }
+        if (comp) mma(cur);
+    };
+    auto tail = [&](int par, const Frag &cur, Frag &nxt) {
+        if (kt + 1 < nk) {
+            landed(max(0, min(nk, kt + NS) - 1 - (kt + C::AHEAD)));
+            if (comp) read(par ^ 1, nxt);
+            if (prod) {
+                if (kt + NS < nk) issue();
+                if (AM == A_F32 && kt + 2 < nk) split(par);
+            }
+        }
+        if (comp) mma(cur);
+    };
+    for (; kt + 1 + NS < nk; kt += 2) {
+        step(0, f0, f1);
+        step(1, f1, f0);
+    }
+    for (; kt < nk; kt++) {
+        tail(0, f0, f1);
+        if (++kt < nk) tail(1, f1, f0);
+    }
+    if (!comp) return;
+    // lane (r, kg) holds rows 4*kg + j, column r of each 16 x 16 block
+#pragma unroll
+    for (int cb = 0; cb < CO; cb++) {
+        const int col = c0 + (wc * CO + cb) * 16 + r;
+        if (col >= (GLU ? g.glu_half : g.N)) continue;
+        const float bc = g.bias ? bf2f(bia[cb]) : 0.0f, bg = GLU && g.bias ? bf2f(bia[cb + (GLU ? CO : 0)]) : 0.0f;
+#pragma unroll
+        for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j;
+                if (m >= g.M || (g.row_mask && !g.row_mask[m])) continue;
+                const float s = acc[rb][cb][j] + bc;
+                if (GLU) {
+                    const float gt = acc[rb][cb + (GLU ? CO : 0)][j] + bg;
+                    g.Y[(long)m * g.ldy + col] = s * sigmoid_hw(gt);
+                } else if (fm) {
+                    g.Y[(long)m * g.ldy + col] = yres[rb][cb][j] + g.scale * s;
+                } else {
+                    store_out(g, m, col, s);
+                }
+            }
+    }
+}
+
+template <class C, bool GLU>
+__global__ __launch_bounds__(64 * C::NW) void gemm_rows_kernel(CtGemm g, int n_mt, int nt) {
+    __shared__ __attribute__((aligned(16))) char smem[C::LDS];
+    const int per = (nt + 7) / 8;
+    const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;   // each XCD takes a range of column tiles
+    if (t >= nt) return;
+    rows_body<C, GLU>(g, t, n_mt, smem);
+}
+
+template <class C>
+void launch_rows_cfg(const CtGemm &g, hipStream_t s) {
+    const bool glu = g.epi == CT_EPI_GLU;
+    const int n_mt = (g.M + C::TM - 1) / C::TM;
+    const int cols = glu ? g.glu_half : g.N, tc = glu ? C::TN / 2 : C::TN;
+    const int nt = n_mt * ((cols + tc - 1) / tc), blocks = (nt + 7) / 8 * 8;
+    if constexpr (C::CB % 2 == 0)
+        if (glu) {
+            hipLaunchKernelGGL((gemm_rows_kernel<C, true>), dim3(blocks), dim3(64 * C::NW), 0, s, g, n_mt, nt);
+            return;
+        }
+    hipLaunchKernelGGL((gemm_rows_kernel<C, false>), dim3(blocks), dim3(64 * C::NW), 0, s, g, n_mt, nt);
+}
+
+// The few-row tiles, smallest first: rows, weight columns, whether the GLU
+// form exists (a wave needs an even number of column blocks), and the
+// measured us per 1000 of K of one workgroup per CU, for A_F32, A_HILO, A_HI.
+struct RowsTile { int tm, tn; bool glu; float us[3]; };
+constexpr RowsTile ROWS_TILES[] = {
+    {16, 16, false, {1.9f, 1.4f, 1.0f}},
+    {16, 32, true, {2.1f, 1.85f, 1.05f}},
+    {32, 32, false, {3.1f, 1.9f, 1.1f}},
+    {32, 64, true, {4.5f, 3.1f, 2.3f}},
+    {64, 128, true, {13.f, 8.4f, 5.6f}},
+};
+constexpr int N_ROWS_TILES = sizeof ROWS_TILES / sizeof ROWS_TILES[0];
+
+template <int AM>
+void launch_rows(int tile, const CtGemm &g, hipStream_t s) {
+    //                                    RB CB WR WC P0 NW  KS NS
+    switch (tile) {
+    case 0: return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 1, 1, 5, 128, 5>>(g, s);
+    case 1:
+        if (g.epi == CT_EPI_GLU) return launch_rows_cfg<RowsCfg<AM, 1, 2, 1, 1, 1, 5, 128, 4>>(g, s);
+        return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 2, 2, 6, 128, 4>>(g, s);
+    case 2: return launch_rows_cfg<RowsCfg<AM, 1, 1, 2, 2, 4, AM == A_F32 ? 12 : 8, 128, 4>>(g, s);
+    case 3: return launch_rows_cfg<RowsCfg<AM, 1, 2, 2, 2, 4, 8, 64, 4>>(g, s);
+    default: return launch_rows_cfg<RowsCfg<AM, 2, 2, 2, 4, 0, 8, 64, AM == A_F32 ? 4 : 3>>(g, s);
+    }
+}
+
 __global__ void split_kernel(uint16_t *hi, uint16_t *lo, const float *x, long n) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -1525,9 +1909,7 @@ static int g_force_tile = 0;
 extern "C" void ctk_gemm_force_tile(int rows) { g_force_tile = rows; }
 extern "C" int ctk_gemm_sizeof(void) { return (int)sizeof(CtGemm); }
 
-// Tile-count model for the two pre-split kernels: a 256-row tile costs about
-// 1.74 128-row tiles (measured), and tiles run in rounds over the CUs.
-static int prefer_256(int M, int n_nt) {
+static int cu_count(void) {
     static int cus = 0;
     if (!cus) {
         int dev = 0;
@@ -1535,9 +1917,53 @@ static int prefer_256(int M, int n_nt) {
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             cus = 256;
     }
+    return cus;
+}
+
+// Tile-count model for the two pre-split kernels: a 256-row tile costs about
+// 1.74 128-row tiles (measured), and tiles run in rounds over the CUs.
+static int prefer_256(int M, int n_nt) {
+    const int cus = cu_count();
     const long t128 = (long)((M + SBM - 1) / SBM) * n_nt, t256 = (long)((M + TBM - 1) / TBM) * n_nt;
     const double r128 = (double)((t128 + cus - 1) / cus), r256 = (double)((t256 + cus - 1) / cus);
     return r256 * 1.74 < r128;
+}
+
+
+// Index of the few-row tile to run, or -1 for the many-row kernels: the lowest
+// estimate of time, from rates measured on the encoder's shapes at 3 to 13056
+// rows (ROWS_TILES; a many-row tile of 128 x 256 takes 21 us per 1000 of K and
+// 8.6 us more, hi + lo).  w: workgroups per CU.  Two small workgroups share a
+// CU at 1.55 times the cost each; the larger tiles run in rounds.  Where the
+// line falls (us, few-row against many-row): 1280 x 5120 hi + lo, 1500 rows
+// 50 against 115, 2700 rows 97 against 118; 3840 x 1280, 1008 rows 34 against
+// 38, 1500 rows 52 against 40.
+static int rows_tile(const CtGemm *g, int am) {
+    const bool glu = g->epi == CT_EPI_GLU;
+    // every DMA address is a base and a 32-bit offset within the tile's rows
+    const long wspan = (long)(glu ? g->glu_half + 256 : 256) * g->K * 2, aspan = 64L * g->lda * 4;
+    if (g->K % 128 || wspan >= 1L << 31 || aspan >= 1L << 31) return -1;
+    const double cus = cu_count(), k = g->K / 1000.0;
+    const int cols = glu ? g->glu_half : g->N;
+    int best = -1;
+    double bt = 0;
+    for (int i = 0; i < N_ROWS_TILES; i++) {
+        const RowsTile &t = ROWS_TILES[i];
+        if (glu && !t.glu) continue;
+        const int tc = glu ? t.tn / 2 : t.tn;
+        const double w = (double)((g->M + t.tm - 1) / t.tm) * ((cols + tc - 1) / tc) / cus;
+        const double us = t.tm == 64 ? ceil(w) * (k * t.us[am] + 5.5)
+                                     : k * t.us[am] * (w <= 1 ? 1 : 1.55 * w) + 1.6 * (w <= 1 ? 1 : w);
+        if (g_force_tile ? g_force_tile == t.tm * 1000 + t.tn : best < 0 || us < bt) { best = i; bt = us; }
+    }
+    if (g_force_tile) return best;
+    const int btn = (am == A_F32 ? 128 : 256) / (glu ? 2 : 1), n_nt = (cols + btn - 1) / btn;
+    const double w = (double)((g->M + 127) / 128) * n_nt / cus;
+    if (am == A_F32) return bt < (w < 1.25 ? 1.25 : w) * (26 * k + 4) ? best : -1;
+    const double one = (am == A_HILO ? 21 : 14) * k + 8.6, w2 = (double)((g->M + 255) / 256) * n_nt / cus;
+    double many = ceil(w) * one;
+    if (g->M >= CT_SPLIT256_MIN_M && 1.74 * ceil(w2) * one < many) many = 1.74 * ceil(w2) * one;
+    return bt < many ? best : -1;
 }
 
 extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
@@ -1554,6 +1980,8 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
             exit(1);
         }
         const bool glu = g->epi == CT_EPI_GLU;
+        const int rt = rows_tile(g, g->Alo ? A_HILO : A_HI);
+        if (rt >= 0) return g->Alo ? launch_rows<A_HILO>(rt, *g, s) : launch_rows<A_HI>(rt, *g, s);
         const int n_mt = (g->M + SBM - 1) / SBM;
         const int n_nt = glu ? (g->glu_half + SBN / 2 - 1) / (SBN / 2) : (g->N + SBN - 1) / SBN;
         const int nt = n_mt * n_nt, per = (nt + 7) / 8;
@@ -1585,6 +2013,8 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
         else hipLaunchKernelGGL(gemm_dec_kernel<1>, grid, dim3(64 * DSPLIT), 0, s, *g);
         return;
     }
+    const int rt = vec ? rows_tile(g, A_F32) : -1;
+    if (rt >= 0) return launch_rows<A_F32>(rt, *g, s);
     if (vec && g->K % BK == 0 && g->M > 64) {
         // same per-element MFMA sequence as the small-M kernels: bit-identical rows
         const int n_mt = (g->M + BT - 1) / BT;

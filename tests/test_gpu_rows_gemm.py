@@ -1,0 +1,95 @@
+"""GPU checks of the few-row encoder GEMM (ctk_gemm's 16- to 64-row tiles):
+every tile gives the bits of the many-row kernels (the same chain of MFMAs per
+element), whatever the rows, columns and depth leave over at the tile's and the
+ring's edges, and writes nothing outside the rows and columns of the launch.
+
+The many-row kernels themselves are held to float64 by test_gpu_split_gemm.py.
+Shapes: rows from 1 past each tile's edge, columns that end inside a tile (a
+multiple of neither 16 nor 8 among them), K from one stage (128) over an odd
+number of stages (384, 640) to one longer than the ring.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import ctbind as cb
+from structs import CtGemm, CtSeg
+from test_gpu_gemv import Dev, f32_to_bf16, split
+
+pytestmark = pytest.mark.gpu
+
+EPI_STORE, EPI_SILU, EPI_RELU, EPI_FMADD, EPI_GLU = 0, 1, 2, 3, 4
+OUT_SPLIT = 3
+TILES = [16016, 16032, 32032, 32064, 64128]
+MANY_ROWS = 128              # forces the many-row kernels
+
+
+@pytest.fixture(scope="module")
+def lib(hip):
+    L = C.CDLL(cb.HIP_LIB)
+    L.ctk_gemm_sizeof.restype = C.c_int
+    assert C.sizeof(CtGemm) == L.ctk_gemm_sizeof()
+    L.ctk_gemm.argtypes = [C.POINTER(CtGemm), C.c_void_p]
+    L.ctk_gemm_force_tile.argtypes = [C.c_int]
+    yield L
+    L.ctk_gemm_force_tile(0)
+
+
+# rows, columns (GLU: of the output), K, epilogue
+SHAPES = [
+    (1, 48, 128, EPI_STORE), (15, 1000, 256, EPI_RELU), (17, 44, 384, EPI_FMADD), (33, 136, 640, EPI_SILU),
+    (65, 200, 1280, EPI_FMADD), (101, 1280, 1280, "split"), (64, 72, 384, EPI_GLU), (100, 640, 1280, EPI_GLU),
+    (13, 1280, 5120, EPI_FMADD),
+]
+
+
+@pytest.mark.parametrize("act", ["fp32", "hilo", "hi"])
+@pytest.mark.parametrize("M,N,K,epi", SHAPES, ids=[f"{m}x{n}x{k}-{e}" for m, n, k, e in SHAPES])
+def test_tiles_give_the_many_row_kernels_bits(lib, hip, act, M, N, K, epi):
+    dev = Dev(hip)
+    rng = np.random.default_rng(M * N + K)
+    glu = epi == EPI_GLU
+    wrows, lda = (2 * N if glu else N), K + 8
+    x = np.zeros((M, lda), np.float32)
+    x[:, :K] = rng.standard_normal((M, K))
+    hi, lo = split(x)
+    pA, pH, pL = dev.put(x), dev.put(hi), dev.put(lo)
+    pW = dev.put(f32_to_bf16(rng.standard_normal((wrows, K)).astype(np.float32) / np.sqrt(K).astype(np.float32)))
+    pb = dev.put(f32_to_bf16(rng.standard_normal(wrows).astype(np.float32)))
+    ldy, guard = N + 8, 3                       # columns and rows past the launch's keep their fill
+    y0 = rng.standard_normal((M + guard, ldy)).astype(np.float32)
+    pY, pY2 = dev.put(y0), dev.put(y0)
+
+    def run(tile):
+        g = CtGemm(lda=lda, W=pW, bias=pb if M != 33 else None, M=M, N=wrows, K=K, scale=0.5, Y=pY, ldy=ldy)
+        if act == "fp32":
+            g.A = pA
+        else:
+            g.Ahi, g.Alo = pH, pL if act == "hilo" else None
+        if epi == "split":
+            g.epi, g.nseg, g.seg_w = EPI_SILU, 1, N
+            g.seg[0] = CtSeg(mode=OUT_SPLIT, base=pY, ld=ldy, base_lo=pY2)
+        else:
+            g.epi = epi
+            g.glu_half = N if glu else 0
+        for p in (pY, pY2):
+            hip.backend_htod(p, y0.ctypes.data, y0.size)
+        dev.ev.sync()
+        lib.ctk_gemm_force_tile(tile)
+        lib.ctk_gemm(C.byref(g), None)
+        return [dev.get(p, np.uint32, y0.size).reshape(y0.shape) for p in (pY, pY2)]
+
+    want = run(MANY_ROWS)
+    for tile in TILES:
+        if glu and tile in (16016, 32032):
+            continue                            # no GLU form: an odd number of column blocks per wave
+        print(f"case: {act} {M}x{N}x{K} epi {epi} tile {tile}", flush=True)
+        got = run(tile)
+        for a, b in zip(want, got):
+            assert np.array_equal(a, b), tile
+    if epi != "split":
+        assert np.array_equal(want[0][M:], y0[M:].view(np.uint32))
+        assert np.array_equal(want[0][:, N:], y0[:, N:].view(np.uint32))
+    for a, b in zip(want, run(0)):              # the tile the cost model takes
+        assert np.array_equal(a, b)
