@@ -170,99 +170,108 @@ __device__ __forceinline__ void store_out8(const CtGemm &g, int m, int col, floa
 
 // ---------------------------------------------------------------------------
 // Decoder-class GEMM (weights with K = 1024, or K = 4096 -> 1024): few rows
-// (one per decode slot), weight-stream bound.  A workgroup owns 16*CB output
-// columns and up to 64 rows; its DSPLIT wavefronts take contiguous K ranges,
-// issue all of their loads early, and the DSPLIT partial tiles are summed in
-// LDS in wave order.  The split depends only on K, never on M, so a row's
-// result is the same for any number of rows.
+// (one per decode slot), bound by the latency of its loads and by what one CU
+// reads.  A workgroup owns 16*RB rows and 16*CB output columns; its DSPLIT
+// wavefronts take contiguous K ranges and the DSPLIT partial tiles are summed
+// in LDS in wave order.  The split depends only on K, never on M, so a row's
+// result is the same for any number of rows.  Row blocks of one column tile
+// run on one XCD (launch position x + y * gridDim.x, gridDim.x a multiple of
+// 8 at the model's sizes), which so fetches the weights once.
+// With the rows split over workgroups, the loads free of branches and a whole
+// group of K-steps in flight (before: one workgroup for 64 rows, two K-steps):
+// 1 row x 4096 x 1024 6.1 -> 4.4 us, 1 x 16384 x 1024 14.2 -> 8.4;
+// 48 rows: 1024 x 1024 9.2 -> 5.4, 4096 x 1024 12 -> 8.8, 1024 x 4096
+// 29 -> 13.8, 16384 x 1024 24.6 -> 21.
 // ---------------------------------------------------------------------------
 #ifndef CT_DEC_SPLIT
 #define CT_DEC_SPLIT 8
 #endif
 constexpr int DSPLIT = CT_DEC_SPLIT;
 
-template <int CB>
+// split_bf16 of eight values, two per conversion instruction
+__device__ __forceinline__ void split8(float4 x0, float4 x1, bf16x8 &hi, bf16x8 &lo) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x[2 * i], x[2 * i + 1]}, bf16x2));
+        const float r0 = x[2 * i] - __uint_as_float(h[i] << 16), r1 = x[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u);
+        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){r0, r1}, bf16x2));
+    }
+    hi = __builtin_bit_cast(bf16x8, h);
+    lo = __builtin_bit_cast(bf16x8, l);
+}
+
+template <int RB, int CB, int KP>
 __global__ __launch_bounds__(64 * DSPLIT) void gemm_dec_kernel(CtGemm g) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, kg = lane >> 4;
     const int c0 = blockIdx.x * 16 * CB;
-    const int m0 = blockIdx.y * 64;
-    const int nrb = min(4, (g.M - m0 + 15) / 16);
+    const int m0 = blockIdx.y * 16 * RB;
     const int kper = g.K / DSPLIT;
-    const int kbeg = w * kper;
-    f32x4 acc[4][CB];
+    const long kbeg = (long)w * kper + kg * 8;
+    f32x4 acc[RB][CB];
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++)
+    for (int rb = 0; rb < RB; rb++)
 #pragma unroll
         for (int cb = 0; cb < CB; cb++) acc[rb][cb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const float *arow[4];
+    // rows and columns past the end re-read the last one: their sums are
+    // never stored, and the loads carry no branch
+    const float *ap[RB];
+    const uint16_t *wp[CB];
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++) {
-        const int m = m0 + rb * 16 + r;
-        arow[rb] = (m < g.M) ? g.A + (long)m * g.lda : nullptr;
-    }
-    const uint16_t *wrow[CB];
+    for (int rb = 0; rb < RB; rb++) ap[rb] = g.A + (long)min(m0 + rb * 16 + r, g.M - 1) * g.lda + kbeg;
 #pragma unroll
-    for (int cb = 0; cb < CB; cb++) {
-        const int n = c0 + cb * 16 + r;
-        wrow[cb] = (n < g.N) ? g.W + (long)n * g.K : nullptr;
-    }
-    for (int k0 = kbeg; k0 < kbeg + kper; k0 += 64) {
-        // two K-steps of loads in flight
-        float4 a[2][4][2];
-        u16x8 wv[2][CB];
+    for (int cb = 0; cb < CB; cb++) wp[cb] = g.W + (long)min(c0 + cb * 16 + r, g.N - 1) * g.K + kbeg;
+    // KP K-steps at a time: every load of the group goes out before its first MFMA
+    struct Group { u16x8 wv[KP][CB]; float4 a[KP][RB][2]; };
+    auto load = [&](int k0, Group &f) {
 #pragma unroll
-        for (int st = 0; st < 2; st++) {
-            const int kk = k0 + st * 32 + kg * 8;
-            const bool ok = kk < kbeg + kper;
+        for (int st = 0; st < KP; st++)
 #pragma unroll
-            for (int rb = 0; rb < 4; rb++) {
-                if (ok && rb < nrb && arow[rb]) {
-                    const float4 *p = reinterpret_cast<const float4 *>(arow[rb] + kk);
-                    a[st][rb][0] = p[0]; a[st][rb][1] = p[1];
-                } else {
-                    a[st][rb][0] = a[st][rb][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-                }
+            for (int cb = 0; cb < CB; cb++) f.wv[st][cb] = *reinterpret_cast<const u16x8 *>(wp[cb] + k0 + st * 32);
+#pragma unroll
+        for (int st = 0; st < KP; st++)
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+                const float4 *p = reinterpret_cast<const float4 *>(ap[rb] + k0 + st * 32);
+                f.a[st][rb][0] = p[0]; f.a[st][rb][1] = p[1];
             }
+    };
+    auto use = [&](const Group &f) {
 #pragma unroll
-            for (int cb = 0; cb < CB; cb++)
-                wv[st][cb] = (ok && wrow[cb]) ? *reinterpret_cast<const u16x8 *>(wrow[cb] + kk)
-                                              : (u16x8){0, 0, 0, 0, 0, 0, 0, 0};
-        }
+        for (int st = 0; st < KP; st++)
 #pragma unroll
-        for (int st = 0; st < 2; st++) {
-            if (k0 + st * 32 >= kbeg + kper) break;
+            for (int rb = 0; rb < RB; rb++) {
+                bf16x8 ah, al;
+                split8(f.a[st][rb][0], f.a[st][rb][1], ah, al);
 #pragma unroll
-            for (int rb = 0; rb < 4; rb++) {
-                if (rb >= nrb) break;
-                const float x[8] = {a[st][rb][0].x, a[st][rb][0].y, a[st][rb][0].z, a[st][rb][0].w,
-                                    a[st][rb][1].x, a[st][rb][1].y, a[st][rb][1].z, a[st][rb][1].w};
-                u16x8 hi, lo;
+                for (int cb = 0; cb < CB; cb++) acc[rb][cb] = mfma16(ah, as_bf16x8(f.wv[st][cb]), acc[rb][cb]);
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    uint16_t h, l;
-                    split_bf16(x[j], h, l);
-                    hi[j] = h; lo[j] = l;
-                }
-                const bf16x8 ah = as_bf16x8(hi), al = as_bf16x8(lo);
-#pragma unroll
-                for (int cb = 0; cb < CB; cb++) {
-                    const bf16x8 bw = as_bf16x8(wv[st][cb]);
-                    acc[rb][cb] = mfma16(ah, bw, acc[rb][cb]);
-                    acc[rb][cb] = mfma16(al, bw, acc[rb][cb]);
-                }
+                for (int cb = 0; cb < CB; cb++) acc[rb][cb] = mfma16(al, as_bf16x8(f.wv[st][cb]), acc[rb][cb]);
             }
-        }
+    };
+    Group f0, f1;
+    load(0, f0);
+    for (int k0 = 0; k0 < kper; k0 += 64 * KP) {
+        if (k0 + 32 * KP < kper) load(k0 + 32 * KP, f1);
+        use(f0);
+        if (k0 + 32 * KP >= kper) break;
+        if (k0 + 64 * KP < kper) load(k0 + 64 * KP, f0);
+        use(f1);
     }
-    __shared__ float part[DSPLIT][64][16 * CB + 1];
+    __shared__ float part[DSPLIT][16 * RB][16 * CB + 1];
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++)
+    for (int rb = 0; rb < RB; rb++)
 #pragma unroll
         for (int cb = 0; cb < CB; cb++)
 #pragma unroll
             for (int j = 0; j < 4; j++) part[w][rb * 16 + kg * 4 + j][cb * 16 + r] = acc[rb][cb][j];
     __syncthreads();
-    for (int e = threadIdx.x; e < 64 * 16 * CB; e += 64 * DSPLIT) {
+    for (int e = threadIdx.x; e < 256 * RB * CB; e += 64 * DSPLIT) {
         const int row = e / (16 * CB), cc = e % (16 * CB);
         const int m = m0 + row, col = c0 + cc;
         if (m >= g.M || col >= g.N) continue;
@@ -273,6 +282,12 @@ __global__ __launch_bounds__(64 * DSPLIT) void gemm_dec_kernel(CtGemm g) {
         if (g.bias) s += bf2f(g.bias[col]);
         store_out(g, m, col, s);
     }
+}
+
+template <int RB, int CB, int KP>
+void launch_dec(const CtGemm &g, hipStream_t s) {
+    hipLaunchKernelGGL((gemm_dec_kernel<RB, CB, KP>), dim3((g.N + 16 * CB - 1) / (16 * CB), (g.M + 16 * RB - 1) / (16 * RB)),
+                       dim3(64 * DSPLIT), 0, s, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -1417,23 +1432,6 @@ __device__ __forceinline__ int rswz(int R, int c) {
     return c ^ (NCH >= 16 ? (R & 15) : ((R & 7) ^ ((R >> 3) & 1)));
 }
 
-// split_bf16 of eight values, two per conversion instruction
-__device__ __forceinline__ void split8(float4 x0, float4 x1, bf16x8 &hi, bf16x8 &lo) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    u32x4 h, l;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x[2 * i], x[2 * i + 1]}, bf16x2));
-        const float r0 = x[2 * i] - __uint_as_float(h[i] << 16), r1 = x[2 * i + 1] - __uint_as_float(h[i] & 0xffff0000u);
-        l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){r0, r1}, bf16x2));
-    }
-    hi = __builtin_bit_cast(bf16x8, h);
-    lo = __builtin_bit_cast(bf16x8, l);
-}
-
 // s_waitcnt vmcnt(y * PW) lgkmcnt(0) for a runtime y <= Y
 template <int Y, int PW>
 __device__ __forceinline__ void wait_younger(int y) {
@@ -2007,10 +2005,17 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
                      (((uintptr_t)g->A & 15) == 0) && (((uintptr_t)g->W & 15) == 0);
     const bool glu = g->epi == CT_EPI_GLU;
     if (vec && decoder_class(g)) {
-        const int cb = g->N >= 4096 ? 2 : 1;
-        const dim3 grid((g->N + 16 * cb - 1) / (16 * cb), (g->M + 63) / 64);
-        if (cb == 2) hipLaunchKernelGGL(gemm_dec_kernel<2>, grid, dim3(64 * DSPLIT), 0, s, *g);
-        else hipLaunchKernelGGL(gemm_dec_kernel<1>, grid, dim3(64 * DSPLIT), 0, s, *g);
+        // The smallest tile whose workgroups all run at once: below that the
+        // weights and activations a CU reads grow, above it a second round
+        // starts.  1024 x 1024 x 48 rows: 16 x 16 5.4 us, 16 x 32 6.5, 32 x 32
+        // 8.2; 4096 x 1024 x 64: 32 x 32 8.8, 16 x 16 14; 16384 x 1024 x 48:
+        // 32 x 64 21, 16 x 64 23.
+        const long nt = (g->N + 15) / 16, mt = (g->M + 15) / 16, cus = cu_count();
+        if (nt * mt <= cus) launch_dec<1, 1, 4>(*g, s);
+        else if ((nt + 1) / 2 * mt <= cus) launch_dec<1, 2, 4>(*g, s);
+        else if (mt > 1 && (nt + 1) / 2 * ((mt + 1) / 2) <= cus) launch_dec<2, 2, 4>(*g, s);
+        else if (mt == 1) launch_dec<1, 4, 4>(*g, s);
+        else launch_dec<2, 4, 2>(*g, s);
         return;
     }
     const int rt = vec ? rows_tile(g, A_F32) : -1;
