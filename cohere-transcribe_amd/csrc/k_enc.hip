@@ -211,10 +211,14 @@ __global__ __launch_bounds__(256) void relpos_attn_kernel(float *O, const float 
 // ---------------------------------------------------------------------------
 // One thread per 8 consecutive channels of DW_RB consecutive rows: the
 // DW_RB + 8 input rows the taps reach are read once (16-byte pieces) and kept
-// in registers, so each input row is fetched about twice instead of once per
-// tap.  The arithmetic per element is the scalar form's (taps in order, taps
-// outside the row's sequence skipped, then BN and SiLU).
-constexpr int DW_RB = 8;
+// in registers.  The arithmetic per element is the scalar form's (taps in
+// order, taps outside the row's sequence skipped, then BN and SiLU).  With few
+// rows the launch is bound by one thread's instructions, so a thread takes a
+// single row; with many, by the rows fetched again by their neighbours, so it
+// takes 8.  us at 101 rows: 8 rows a thread 12.1, 4 8.4, 2 5.8, 1 4.7; at 1008
+// 12.4, 9.4, 8.2, 7.8; at 2600 14.8, 14.4, 16.6, 18.1; at 13000 53, 54, 63, 72.
+constexpr int DW_ROWS_FEW = 1600;
+template <int DW_RB>
 __global__ __launch_bounds__(256) void dwconv_bn_silu_kernel(float *out, uint16_t *out_hi, uint16_t *out_lo,
                                                              const float *in, int M, const int *row_start,
                                                              const int *row_len, const uint16_t *dww,
@@ -588,13 +592,23 @@ extern "C" void ctk_relpos_attn_packed(float *O, uint16_t *Oh, uint16_t *Ol, con
                        O, Q, K, V, P, pbu, pbv, 0, T_max, seq_off, seq_T, blk_seq, blk_q0, ldS, Oh, Ol);
 }
 
+static void launch_dwconv(float *out, uint16_t *out_hi, uint16_t *out_lo, const float *in, int M, const int *row_start,
+                          const int *row_len, const uint16_t *dww, const uint16_t *dwb, const uint16_t *bnw,
+                          const uint16_t *bnb, const uint16_t *bnm, const uint16_t *bnv, hipStream_t s) {
+    if (M <= DW_ROWS_FEW)
+        hipLaunchKernelGGL(dwconv_bn_silu_kernel<1>, dim3(nblk((long)M * (ENC_D / 8))), dim3(256), 0, s, out, out_hi,
+                           out_lo, in, M, row_start, row_len, dww, dwb, bnw, bnb, bnm, bnv);
+    else
+        hipLaunchKernelGGL(dwconv_bn_silu_kernel<8>, dim3(nblk((long)((M + 7) / 8) * (ENC_D / 8))), dim3(256), 0, s, out,
+                           out_hi, out_lo, in, M, row_start, row_len, dww, dwb, bnw, bnb, bnm, bnv);
+}
+
 extern "C" void ctk_dwconv_bn_silu(float *out, const float *in, int T, const uint16_t *dww,
                                    const uint16_t *dwb, const uint16_t *bnw, const uint16_t *bnb,
                                    const uint16_t *bnm, const uint16_t *bnv, hipStream_t s) {
     if (T <= 0) return;
     dw_check(out, nullptr, in, dww, dwb, bnw, bnb, bnm, bnv);
-    hipLaunchKernelGGL(dwconv_bn_silu_kernel, dim3(nblk((long)((T + DW_RB - 1) / DW_RB) * (ENC_D / 8))), dim3(256), 0, s,
-                       out, nullptr, nullptr, in, T, nullptr, nullptr, dww, dwb, bnw, bnb, bnm, bnv);
+    launch_dwconv(out, nullptr, nullptr, in, T, nullptr, nullptr, dww, dwb, bnw, bnb, bnm, bnv, s);
 }
 
 extern "C" void ctk_dwconv_bn_silu_packed(uint16_t *out_hi, uint16_t *out_lo, const float *in, int M,
@@ -605,8 +619,7 @@ extern "C" void ctk_dwconv_bn_silu_packed(uint16_t *out_hi, uint16_t *out_lo, co
     if (M <= 0) return;
     dw_check(nullptr, out_hi, in, dww, dwb, bnw, bnb, bnm, bnv);
     if ((uintptr_t)out_lo & 15) { fprintf(stderr, "dwconv: outputs must be 16-byte aligned\n"); exit(1); }
-    hipLaunchKernelGGL(dwconv_bn_silu_kernel, dim3(nblk((long)((M + DW_RB - 1) / DW_RB) * (ENC_D / 8))), dim3(256), 0, s,
-                       nullptr, out_hi, out_lo, in, M, row_start, row_len, dww, dwb, bnw, bnb, bnm, bnv);
+    launch_dwconv(nullptr, out_hi, out_lo, in, M, row_start, row_len, dww, dwb, bnw, bnb, bnm, bnv, s);
 }
 
 extern "C" void ctk_sub_conv0(float *out, const float *mel, int T_mel, int stride,
