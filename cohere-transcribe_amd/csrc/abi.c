@@ -238,14 +238,19 @@ void backend_layernorm(float *dst, const float *src, const uint16_t *w, const ui
     ctk_layernorm(dst, src, CT_W(w), CT_W(b), T, D, ct_t.stream);
 }
 
+static void linear_args(CtGemm *g, float *y, const float *x, const uint16_t *W, const uint16_t *b,
+                        int T, int in_d, int out_d, int epi, float scale) {
+    memset(g, 0, sizeof *g);
+    g->A = x; g->lda = in_d; g->W = CT_W(W); g->bias = CT_W(b);
+    g->Y = y; g->ldy = out_d; g->M = T; g->N = out_d; g->K = in_d;
+    g->epi = epi; g->scale = scale;
+}
+
 static void linear_epi(float *y, const float *x, const uint16_t *W, const uint16_t *b,
                        int T, int in_d, int out_d, int epi, float scale) {
     require_init();
     CtGemm g;
-    memset(&g, 0, sizeof g);
-    g.A = x; g.lda = in_d; g.W = CT_W(W); g.bias = CT_W(b);
-    g.Y = y; g.ldy = out_d; g.M = T; g.N = out_d; g.K = in_d;
-    g.epi = epi; g.scale = scale;
+    linear_args(&g, y, x, W, b, T, in_d, out_d, epi, scale);
     ctk_gemm(&g, ct_t.stream);
 }
 
@@ -316,8 +321,10 @@ void backend_rel_pos_mhsa(float *x, const float *pos_emb, int T, const ELayer *L
     float *Ys[4] = {Q, K, V, P};
     const uint16_t *Ws[4] = {L->sa_qw, L->sa_kw, L->sa_vw, L->sa_pw};
     const uint16_t *Bs[4] = {L->sa_qb, L->sa_kb, L->sa_vb, NULL};
+    CtGemm g[4];
     for (int i = 0; i < 4; i++)
-        backend_linear(Ys[i], Xs[i], Ws[i], Bs[i], i == 3 ? 2 * T - 1 : T, ENC_D, ENC_D);
+        linear_args(&g[i], Ys[i], Xs[i], Ws[i], Bs[i], i == 3 ? 2 * T - 1 : T, ENC_D, ENC_D, CT_EPI_STORE, 0.0f);
+    ctk_gemm_group(g, 4, ct_t.stream);
     ctk_relpos_attn(O, Q, K, V, P, CT_W(L->sa_pbu), CT_W(L->sa_pbv), T, ct_t.stream);
     backend_linear(x, O, L->sa_ow, L->sa_ob, T, ENC_D, ENC_D);
 }

@@ -66,6 +66,9 @@ typedef struct {
 } CtGemm;
 
 void ctk_gemm(const CtGemm *g, hipStream_t s);
+/* n products that do not depend on each other, in one launch where they can be. */
+#define CT_GEMM_GROUP 4
+void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s);
 /* Tests: 128 or 256 forces the pre-split kernels' tile, rows * 1000 + columns
  * a few-row tile (16016, 16032, 32032, 32064, 64128; 0: the cost model);
  * sizeof(CtGemm) for the tests' struct mirror. */

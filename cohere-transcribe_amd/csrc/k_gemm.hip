@@ -1697,12 +1697,34 @@ __global__ __launch_bounds__(64 * C::NW) void gemm_rows_kernel(CtGemm g, int n_m
     rows_body<C, GLU>(g, t, n_mt, smem);
 }
 
+// Several products in one launch: blockIdx.y picks the product, blockIdx.x its tile.
+struct CtGemmGroup { CtGemm g[CT_GEMM_GROUP]; };
 template <class C>
-void launch_rows_cfg(const CtGemm &g, hipStream_t s) {
+__global__ __launch_bounds__(64 * C::NW) void gemm_rows_group_kernel(CtGemmGroup grp) {
+    __shared__ __attribute__((aligned(16))) char smem[C::LDS];
+    const CtGemm &g = grp.g[blockIdx.y];
+    const int n_mt = (g.M + C::TM - 1) / C::TM, nt = n_mt * ((g.N + C::TN - 1) / C::TN), per = (nt + 7) / 8;
+    if ((int)blockIdx.x >= 8 * per) return;
+    const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (t >= nt) return;
+    rows_body<C, false>(g, t, n_mt, smem);
+}
+
+template <class C>
+void launch_rows_cfg(const CtGemm &g, hipStream_t s, const CtGemmGroup *grp, int n) {
     const bool glu = g.epi == CT_EPI_GLU;
-    const int n_mt = (g.M + C::TM - 1) / C::TM;
-    const int cols = glu ? g.glu_half : g.N, tc = glu ? C::TN / 2 : C::TN;
-    const int nt = n_mt * ((cols + tc - 1) / tc), blocks = (nt + 7) / 8 * 8;
+    auto tiles = [&](const CtGemm &q) {
+        const int cols = glu ? q.glu_half : q.N, tc = glu ? C::TN / 2 : C::TN;
+        return (q.M + C::TM - 1) / C::TM * ((cols + tc - 1) / tc);
+    };
+    if constexpr (C::AM == A_F32)
+        if (grp) {
+            int nt = 0;
+            for (int i = 0; i < n; i++) nt = max(nt, tiles(grp->g[i]));
+            hipLaunchKernelGGL(gemm_rows_group_kernel<C>, dim3((nt + 7) / 8 * 8, n), dim3(64 * C::NW), 0, s, *grp);
+            return;
+        }
+    const int n_mt = (g.M + C::TM - 1) / C::TM, nt = tiles(g), blocks = (nt + 7) / 8 * 8;
     if constexpr (C::CB % 2 == 0)
         if (glu) {
             hipLaunchKernelGGL((gemm_rows_kernel<C, true>), dim3(blocks), dim3(64 * C::NW), 0, s, g, n_mt, nt);
@@ -1724,17 +1746,18 @@ constexpr RowsTile ROWS_TILES[] = {
 };
 constexpr int N_ROWS_TILES = sizeof ROWS_TILES / sizeof ROWS_TILES[0];
 
+// grp: the n products of a group launch (g the first of them)
 template <int AM>
-void launch_rows(int tile, const CtGemm &g, hipStream_t s) {
+void launch_rows(int tile, const CtGemm &g, hipStream_t s, const CtGemmGroup *grp = nullptr, int n = 1) {
     //                                    RB CB WR WC P0 NW  KS NS
     switch (tile) {
-    case 0: return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 1, 1, 5, 128, 5>>(g, s);
+    case 0: return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 1, 1, 5, 128, 5>>(g, s, grp, n);
     case 1:
-        if (g.epi == CT_EPI_GLU) return launch_rows_cfg<RowsCfg<AM, 1, 2, 1, 1, 1, 5, 128, 4>>(g, s);
-        return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 2, 2, 6, 128, 4>>(g, s);
-    case 2: return launch_rows_cfg<RowsCfg<AM, 1, 1, 2, 2, 4, AM == A_F32 ? 12 : 8, 128, 4>>(g, s);
-    case 3: return launch_rows_cfg<RowsCfg<AM, 1, 2, 2, 2, 4, 8, 64, 4>>(g, s);
-    default: return launch_rows_cfg<RowsCfg<AM, 2, 2, 2, 4, 0, 8, 64, AM == A_F32 ? 4 : 3>>(g, s);
+        if (g.epi == CT_EPI_GLU) return launch_rows_cfg<RowsCfg<AM, 1, 2, 1, 1, 1, 5, 128, 4>>(g, s, grp, n);
+        return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 2, 2, 6, 128, 4>>(g, s, grp, n);
+    case 2: return launch_rows_cfg<RowsCfg<AM, 1, 1, 2, 2, 4, AM == A_F32 ? 12 : 8, 128, 4>>(g, s, grp, n);
+    case 3: return launch_rows_cfg<RowsCfg<AM, 1, 2, 2, 2, 4, 8, 64, 4>>(g, s, grp, n);
+    default: return launch_rows_cfg<RowsCfg<AM, 2, 2, 2, 4, 0, 8, 64, AM == A_F32 ? 4 : 3>>(g, s, grp, n);
     }
 }
 
@@ -1928,7 +1951,8 @@ static int prefer_256(int M, int n_nt) {
 }
 
 
-// Index of the few-row tile to run, or -1 for the many-row kernels: the lowest
+// Index of the few-row tile to run n products of one K in one launch (all but
+// the first: no GLU), or -1 for the many-row kernels: the lowest
 // estimate of time, from rates measured on the encoder's shapes at 3 to 13056
 // rows (ROWS_TILES; a many-row tile of 128 x 256 takes 21 us per 1000 of K and
 // 8.6 us more, hi + lo).  w: workgroups per CU.  Two small workgroups share a
@@ -1936,29 +1960,33 @@ static int prefer_256(int M, int n_nt) {
 // line falls (us, few-row against many-row): 1280 x 5120 hi + lo, 1500 rows
 // 50 against 115, 2700 rows 97 against 118; 3840 x 1280, 1008 rows 34 against
 // 38, 1500 rows 52 against 40.
-static int rows_tile(const CtGemm *g, int am) {
+static int rows_tile(const CtGemm *g, int am, int n = 1) {
     const bool glu = g->epi == CT_EPI_GLU;
+    auto wgs = [&](int tm, int tc) {
+        double t = 0;
+        for (int i = 0; i < n; i++)
+            t += (double)((g[i].M + tm - 1) / tm) * (((glu ? g->glu_half : g[i].N) + tc - 1) / tc);
+        return t / cu_count();
+    };
     // every DMA address is a base and a 32-bit offset within the tile's rows
     const long wspan = (long)(glu ? g->glu_half + 256 : 256) * g->K * 2, aspan = 64L * g->lda * 4;
     if (g->K % 128 || wspan >= 1L << 31 || aspan >= 1L << 31) return -1;
-    const double cus = cu_count(), k = g->K / 1000.0;
-    const int cols = glu ? g->glu_half : g->N;
+    const double k = g->K / 1000.0;
     int best = -1;
     double bt = 0;
     for (int i = 0; i < N_ROWS_TILES; i++) {
         const RowsTile &t = ROWS_TILES[i];
         if (glu && !t.glu) continue;
-        const int tc = glu ? t.tn / 2 : t.tn;
-        const double w = (double)((g->M + t.tm - 1) / t.tm) * ((cols + tc - 1) / tc) / cus;
+        const double w = wgs(t.tm, glu ? t.tn / 2 : t.tn);
         const double us = t.tm == 64 ? ceil(w) * (k * t.us[am] + 5.5)
                                      : k * t.us[am] * (w <= 1 ? 1 : 1.55 * w) + 1.6 * (w <= 1 ? 1 : w);
         if (g_force_tile ? g_force_tile == t.tm * 1000 + t.tn : best < 0 || us < bt) { best = i; bt = us; }
     }
     if (g_force_tile) return best;
-    const int btn = (am == A_F32 ? 128 : 256) / (glu ? 2 : 1), n_nt = (cols + btn - 1) / btn;
-    const double w = (double)((g->M + 127) / 128) * n_nt / cus;
+    const int btn = (am == A_F32 ? 128 : 256) / (glu ? 2 : 1);
+    const double w = wgs(128, btn);
     if (am == A_F32) return bt < (w < 1.25 ? 1.25 : w) * (26 * k + 4) ? best : -1;
-    const double one = (am == A_HILO ? 21 : 14) * k + 8.6, w2 = (double)((g->M + 255) / 256) * n_nt / cus;
+    const double one = (am == A_HILO ? 21 : 14) * k + 8.6, w2 = wgs(256, btn);
     double many = ceil(w) * one;
     if (g->M >= CT_SPLIT256_MIN_M && 1.74 * ceil(w2) * one < many) many = 1.74 * ceil(w2) * one;
     return bt < many ? best : -1;
@@ -2033,6 +2061,27 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
     }
     if (vec) { if (glu) dispatch<true, true>(*g, s); else dispatch<true, false>(*g, s); }
     else     { if (glu) dispatch<false, true>(*g, s); else dispatch<false, false>(*g, s); }
+}
+
+// Products of fp32 activations and one K that do not depend on each other: in
+// one launch where they take a few-row tile together, else one by one.  The
+// four projections of relative-position attention (Q, K, V of T rows, P of
+// 2T - 1) as one launch: 7.8 us at T = 13 (6.6 each alone), 16 at 101 (8 and
+// 11), 41 at 376 (11 and 22).
+extern "C" void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s) {
+    bool one = n > 1 && n <= CT_GEMM_GROUP;
+    for (int i = 0; one && i < n; i++)
+        one = g[i].M > 0 && g[i].N > 0 && !g[i].Ahi && g[i].epi != CT_EPI_GLU && g[i].K == g->K && g[i].lda % 4 == 0 &&
+              ((uintptr_t)g[i].A & 15) == 0 && ((uintptr_t)g[i].W & 15) == 0 && !decoder_class(&g[i]) &&
+              rows_tile(&g[i], A_F32) >= 0;       // its own address spans too
+    const int rt = one ? rows_tile(g, A_F32, n) : -1;
+    if (rt < 0) {
+        for (int i = 0; i < n; i++) ctk_gemm(&g[i], s);
+        return;
+    }
+    CtGemmGroup grp;
+    for (int i = 0; i < CT_GEMM_GROUP; i++) grp.g[i] = g[i < n ? i : 0];
+    launch_rows<A_F32>(rt, grp.g[0], s, &grp, n);
 }
 
 extern "C" void ctk_split(uint16_t *hi, uint16_t *lo, const float *x, long n, hipStream_t s) {

@@ -93,3 +93,37 @@ def test_tiles_give_the_many_row_kernels_bits(lib, hip, act, M, N, K, epi):
         assert np.array_equal(want[0][:, N:], y0[:, N:].view(np.uint32))
     for a, b in zip(want, run(0)):              # the tile the cost model takes
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rows,K", [((13, 13, 13, 25), 1280), ((101, 40), 1280), ((376, 376, 1), 384),
+                                    ((20, 31), 1312), ((5,), 256)],
+                         ids=["13", "two", "uneven", "K-not-grouped", "one"])
+def test_group_gives_the_single_launches_bits(lib, hip, rows, K):
+    """ctk_gemm_group: the bits of each product launched alone, its rows past M
+    untouched (K = 1312 has no few-row tile: the group falls back to single launches)."""
+    dev = Dev(hip)
+    lib.ctk_gemm_force_tile(0)
+    lib.ctk_gemm_group.argtypes = [C.POINTER(CtGemm), C.c_int, C.c_void_p]
+    rng = np.random.default_rng(sum(rows) + K)
+    N = 320
+    gs, gs1 = (CtGemm * len(rows))(), (CtGemm * len(rows))()
+    outs = []
+    for i, M in enumerate(rows):
+        px = dev.put(rng.standard_normal((M, K)).astype(np.float32))
+        pW = dev.put(f32_to_bf16(rng.standard_normal((N, K)).astype(np.float32)))
+        pb = dev.put(f32_to_bf16(rng.standard_normal(N).astype(np.float32)))
+        y0 = rng.standard_normal((M + 2, N)).astype(np.float32)
+        py = [dev.put(y0), dev.put(y0)]
+        outs.append((py, y0))
+        for arr, p in ((gs, py[0]), (gs1, py[1])):
+            arr[i] = CtGemm(A=px, lda=K, W=pW, bias=pb if i % 2 == 0 else None, Y=p, ldy=N, M=M, N=N, K=K,
+                            epi=EPI_FMADD if i % 3 == 1 else EPI_STORE, scale=0.5)
+    dev.ev.sync()
+    print(f"case: group of {rows} rows, K {K}", flush=True)
+    lib.ctk_gemm_group(gs, len(rows), None)
+    for i in range(len(rows)):
+        lib.ctk_gemm(C.byref(gs1[i]), None)
+    for (a, b), y0 in outs:
+        got, want = dev.get(a, np.uint32, y0.size).reshape(y0.shape), dev.get(b, np.uint32, y0.size).reshape(y0.shape)
+        assert np.array_equal(got, want)
+        assert np.array_equal(got[-2:], y0[-2:].view(np.uint32))
