@@ -287,19 +287,45 @@ void backend_encoder_subsampling(const float *mel, int T_mel, int T_mel_stride,
     const int T1 = (T_mel + 1) / 2, T2 = (T1 + 1) / 2;
     float *ra = work, *rb = work + (size_t)SUB_CH * T1 * 64;
     hipStream_t s = ct_t.stream;
-    ctk_sub_conv0(ra, mel, T_mel, T_mel_stride, CT_W(W->s0w), CT_W(W->s0b), s);
-    ctk_sub_dwconv(rb, ra, T1, 64, CT_W(W->s2w), CT_W(W->s2b), s);
+    const uint16_t *w1 = CT_W(W->s3w), *w2 = CT_W(W->s6w), *w3 = CT_W(W->sow);
     CtGemm g;
     memset(&g, 0, sizeof g);
-    g.A = rb; g.lda = SUB_CH; g.W = CT_W(W->s3w); g.bias = CT_W(W->s3b);
+    if ((((uintptr_t)work | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)w3) & 15) == 0) {
+        /* Every product's input written as bf16 planes hi, lo in region B (a
+         * stage's floats and its two planes take the same bytes): the first
+         * two convolutions in one pass, and no product splits fp32 rows.  The
+         * bits are those of the stages below. */
+        uint16_t *h = (uint16_t *)rb;
+        size_t n = (size_t)T2 * 32 * SUB_CH;
+        ctk_sub_conv0_dw(h, h + n, mel, T_mel, T_mel_stride, CT_W(W->s0w), CT_W(W->s0b), CT_W(W->s2w),
+                         CT_W(W->s2b), s);
+        g.Ahi = h; g.Alo = h + n; g.lda = SUB_CH; g.W = w1; g.bias = CT_W(W->s3b);
+        g.Y = ra; g.ldy = SUB_CH; g.M = T2 * 32; g.N = SUB_CH; g.K = SUB_CH; g.epi = CT_EPI_RELU;
+        ctk_gemm(&g, s);
+        n = (size_t)((T2 + 1) / 2) * 16 * SUB_CH;
+        ctk_sub_dw_split(h, h + n, ra, T2, 32, CT_W(W->s5w), CT_W(W->s5b), s);
+        g.Alo = h + n; g.W = w2; g.bias = CT_W(W->s6b); g.M = T_enc * 16;
+        ctk_gemm(&g, s);
+        n = (size_t)T_enc * 16 * SUB_CH;
+        ctk_sub_flatten_split(h, h + n, ra, T_enc, s);
+        g.Alo = h + n;
+        g.lda = SUB_CH * 16; g.W = w3; g.bias = CT_W(W->sob);
+        g.Y = x_enc; g.ldy = ENC_D; g.M = T_enc; g.N = ENC_D; g.K = SUB_CH * 16; g.epi = CT_EPI_STORE;
+        ctk_gemm(&g, s);
+        return;
+    }
+    /* scratch or weights off 16 bytes: fp32 stages */
+    ctk_sub_conv0(ra, mel, T_mel, T_mel_stride, CT_W(W->s0w), CT_W(W->s0b), s);
+    ctk_sub_dwconv(rb, ra, T1, 64, CT_W(W->s2w), CT_W(W->s2b), s);
+    g.A = rb; g.lda = SUB_CH; g.W = w1; g.bias = CT_W(W->s3b);
     g.Y = ra; g.ldy = SUB_CH; g.M = T2 * 32; g.N = SUB_CH; g.K = SUB_CH; g.epi = CT_EPI_RELU;
     ctk_gemm(&g, s);
     ctk_sub_dwconv(rb, ra, T2, 32, CT_W(W->s5w), CT_W(W->s5b), s);
-    g.A = rb; g.W = CT_W(W->s6w); g.bias = CT_W(W->s6b); g.Y = ra; g.M = T_enc * 16;
+    g.A = rb; g.W = w2; g.bias = CT_W(W->s6b); g.Y = ra; g.M = T_enc * 16;
     ctk_gemm(&g, s);
     ctk_sub_flatten(rb, ra, T_enc, s);
     memset(&g, 0, sizeof g);
-    g.A = rb; g.lda = SUB_CH * 16; g.W = CT_W(W->sow); g.bias = CT_W(W->sob);
+    g.A = rb; g.lda = SUB_CH * 16; g.W = w3; g.bias = CT_W(W->sob);
     g.Y = x_enc; g.ldy = ENC_D; g.M = T_enc; g.N = ENC_D; g.K = SUB_CH * 16; g.epi = CT_EPI_STORE;
     ctk_gemm(&g, s);
 }

@@ -335,7 +335,13 @@ void ctk_sub_conv0_dw_packed(uint16_t *out_hi, uint16_t *out_lo, const float *me
 void ctk_sub_dw_split_packed(uint16_t *out_hi, uint16_t *out_lo, const float *in, const int *oin,
                              const int *oout, int n, int rows_out, int Wd, const uint16_t *w,
                              const uint16_t *b, hipStream_t s);
-/* The same, written as hi/lo bf16 planes (row stride 4096). */
+/* The two stages for one clip (mel row stride given), without tables. */
+void ctk_sub_conv0_dw(uint16_t *out_hi, uint16_t *out_lo, const float *mel, int T_mel, int stride,
+                      const uint16_t *w0, const uint16_t *b0, const uint16_t *wd, const uint16_t *bd,
+                      hipStream_t s);
+void ctk_sub_dw_split(uint16_t *out_hi, uint16_t *out_lo, const float *in, int H, int Wd, const uint16_t *w,
+                      const uint16_t *b, hipStream_t s);
+/* ctk_sub_flatten, written as hi/lo bf16 planes (row stride 4096). */
 void ctk_sub_flatten_split(uint16_t *hi, uint16_t *lo, const float *in, int T, hipStream_t s);
 
 /* ---------------- log-mel front-end ---------------- */

@@ -366,106 +366,142 @@ __device__ __forceinline__ int packed_owner(const int *off, int n, int tau) {
 // The first two subsampling stages fused, over several requests packed
 // along time: conv 3x3 stride 2 (1 -> 256 channels, ReLU) then depthwise
 // 3x3 stride 2, without storing the conv output.  Workgroup = one output row
-// tau of the depthwise stage (request r, row oh = tau - o2[r]), thread =
-// channel c, looping over the 32 output columns.  The 7 mel frames the row
-// needs (4*oh - 3 .. 4*oh + 3, all 128 bins) are staged in LDS; each conv
-// value a depthwise tap needs is recomputed from them (9 products), in the
-// same order and with the same skips as sub_conv0 then sub_dwconv, so the
-// result is bit-identical to running the two stages
-// (backends/cpu/backend.c:201-221).  The output is written split hi/lo for
-// the pointwise GEMM that reads it.
-constexpr int C0D_FRAMES = 7;
+// tau of the depthwise stage (request r, row oh = tau - o2[r]; without tables,
+// one request of T_arg frames) and SUB_SEG of its 32 output columns, thread =
+// channel c.  The 7 mel frames the row needs (4*oh - 3 .. 4*oh + 3) are staged
+// in LDS frame-contiguous, zero outside the clip, so a thread fetches a bin's
+// 7 frames as two 16-byte broadcasts.
+// Going along the columns, a thread keeps the conv column its next output
+// shares with this one and a mel bin: 6 conv values and 4 bins an output,
+// where computing every tap's conv value takes 9 values and 81 LDS reads.  It
+// is bound by its multiply-adds (63 an output and channel).  Every value is
+// summed in the order of sub_conv0 then sub_dwconv (taps in order; a tap
+// outside adds zero), so with finite weights the result is bit-identical to
+// running the two stages (backends/cpu/backend.c:201-221).  The output is
+// written split hi/lo for the pointwise GEMM that reads it.
+// 24 clips (4134 rows) 199 -> 77 us; one clip of 10 s (251 rows) 11.6, where
+// the two stages took 60.
+constexpr int SUB_SEG = 8;                        // output columns of a workgroup
 __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_hi, uint16_t *out_lo,
                                                                   const float *mel,
                                                                   const int *o1, const int *o2,
                                                                   const int *tmel, const int *moff, int n,
+                                                                  int T_arg, int stride_arg,
                                                                   const uint16_t *w0, const uint16_t *b0,
                                                                   const uint16_t *wd, const uint16_t *bd) {
-    __shared__ float sm[C0D_FRAMES][N_MELS];
-    const int tau = blockIdx.x, c = threadIdx.x;
-    const int r = packed_owner(o2, n, tau);
-    const int oh = tau - o2[r], H1 = o1[r + 1] - o1[r], T_mel = tmel[r];
-    const float *m = mel + moff[r];
-    const int f0 = 4 * oh - 3;                 // first mel frame of the window
-    for (int e = c; e < C0D_FRAMES * N_MELS; e += 256) {
-        const int fr = e / N_MELS, bin = e % N_MELS, ih0 = f0 + fr;
-        sm[fr][bin] = (ih0 >= 0 && ih0 < T_mel) ? m[(long)bin * T_mel + ih0] : 0.0f;
+    constexpr int NB = 4 * SUB_SEG + 3;           // bins 4*ow0 - 3 .. 4*ow0 + 4*SUB_SEG - 1
+    __shared__ float4 sm[NB][2];
+    const int tau = blockIdx.x, c = threadIdx.x, ow0 = blockIdx.y * SUB_SEG;
+    const int r = o2 ? packed_owner(o2, n, tau) : 0;
+    const int oh = o2 ? tau - o2[r] : tau;
+    const int T_mel = o2 ? tmel[r] : T_arg, H1 = o2 ? o1[r + 1] - o1[r] : (T_arg + 1) / 2;
+    const long stride = o2 ? T_mel : stride_arg;
+    const float *m = mel + (o2 ? moff[r] : 0);
+    const int f0 = 4 * oh - 3;                    // first mel frame of the window
+    for (int e = c; e < NB * 8; e += 256) {
+        const int bin = 4 * ow0 - 3 + e / 8, f = f0 + e % 8;
+        reinterpret_cast<float *>(sm)[e] =
+            (e % 8 < 7 && bin >= 0 && bin < N_MELS && f >= 0 && f < T_mel) ? m[bin * stride + f] : 0.0f;
     }
     float k0[9], kd[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) { k0[k] = bf2f(w0[c * 9 + k]); kd[k] = bf2f(wd[c * 9 + k]); }
     const float bias0 = bf2f(b0[c]), biasd = bf2f(bd[c]);
     __syncthreads();
-    const long orow = (long)tau * 32 * SUB_CH + c;
-    for (int ow = 0; ow < 32; ow++) {
+    struct Bin { float f[8]; };
+    auto bin = [&](int i) {                       // bin 4*ow0 - 3 + i
+        Bin b;
+        const float4 x = sm[i][0], y = sm[i][1];
+        b.f[0] = x.x; b.f[1] = x.y; b.f[2] = x.z; b.f[3] = x.w;
+        b.f[4] = y.x; b.f[5] = y.y; b.f[6] = y.z; b.f[7] = y.w;
+        return b;
+    };
+    // the three conv values of one column (rows 2*oh - 1 .. 2*oh + 1) from its
+    // three bins; zero in rows outside the conv output
+    struct Col { float v[3]; };
+    auto conv = [&](const Bin &x0, const Bin &x1, const Bin &x2) {
+        Col q;
+#pragma unroll
+        for (int kh2 = 0; kh2 < 3; kh2++) {
+            const int ih1 = 2 * oh - 1 + kh2;
+            float x = bias0;
+#pragma unroll
+            for (int kh = 0; kh < 3; kh++) {
+                x += x0.f[2 * kh2 + kh] * k0[kh * 3];
+                x += x1.f[2 * kh2 + kh] * k0[kh * 3 + 1];
+                x += x2.f[2 * kh2 + kh] * k0[kh * 3 + 2];
+            }
+            q.v[kh2] = ih1 >= 0 && ih1 < H1 && x > 0.0f ? x : 0.0f;
+        }
+        return q;
+    };
+    Bin last = bin(2);                            // bin 4*ow - 1
+    Col left = conv(bin(0), bin(1), last);        // conv column 2*ow - 1
+    if (ow0 == 0) left.v[0] = left.v[1] = left.v[2] = 0.0f;
+    const long orow = ((long)tau * 32 + ow0) * SUB_CH + c;
+#pragma unroll 2
+    for (int j = 0; j < SUB_SEG; j++) {
+        const Bin x1 = bin(4 * j + 3), x2 = bin(4 * j + 4), x3 = bin(4 * j + 5), x4 = bin(4 * j + 6);
+        const Col mid = conv(last, x1, x2), right = conv(x2, x3, x4);
         float acc = biasd;
 #pragma unroll
         for (int kh2 = 0; kh2 < 3; kh2++) {
-            const int ih1 = oh * 2 - 1 + kh2;
-            if (ih1 < 0 || ih1 >= H1) continue;
-#pragma unroll
-            for (int kw2 = 0; kw2 < 3; kw2++) {
-                const int iw1 = ow * 2 - 1 + kw2;
-                if (iw1 < 0 || iw1 >= 64) continue;
-                // conv value at (ih1, iw1, c)
-                float x = bias0;
-#pragma unroll
-                for (int kh = 0; kh < 3; kh++) {
-                    const int ih0 = ih1 * 2 - 1 + kh;
-                    if (ih0 < 0 || ih0 >= T_mel) continue;
-#pragma unroll
-                    for (int kw = 0; kw < 3; kw++) {
-                        const int iw0 = iw1 * 2 - 1 + kw;
-                        if (iw0 < 0 || iw0 >= N_MELS) continue;
-                        x += sm[ih0 - f0][iw0] * k0[kh * 3 + kw];
-                    }
-                }
-                x = x > 0.0f ? x : 0.0f;
-                acc += x * kd[kh2 * 3 + kw2];
-            }
+            acc += left.v[kh2] * kd[kh2 * 3];
+            acc += mid.v[kh2] * kd[kh2 * 3 + 1];
+            acc += right.v[kh2] * kd[kh2 * 3 + 2];
         }
         uint16_t hh, ll;
         split_bf16(acc, hh, ll);
-        out_hi[orow + (long)ow * SUB_CH] = hh;
-        out_lo[orow + (long)ow * SUB_CH] = ll;
+        out_hi[orow + (long)j * SUB_CH] = hh;
+        out_lo[orow + (long)j * SUB_CH] = ll;
+        left = right;
+        last = x4;
     }
 }
 
 // sub_dwconv_kernel over several requests, written split hi/lo for the
 // pointwise GEMM: request r's input rows oin[r] .. oin[r + 1] of
 // [sum H][Wd][256], output rows oout[r] .. oout[r + 1] of
-// [sum (H+1)/2][(Wd+1)/2][256].  Workgroup = one output row, thread =
-// channel, looping over the output columns; each sum is the scalar form's
-// (taps in order, skips at the edges).
+// [sum (H+1)/2][(Wd+1)/2][256] (without tables, one request of H_arg rows).
+// Workgroup = one output row and SUB_SEG of its columns, thread = channel: the
+// 2*SUB_SEG + 1 input columns of the three rows all in flight at once, each
+// read once; each sum is the scalar form's order (taps outside add zero).
+// 24 clips (2071 rows) 91 -> 36 us.
 __global__ __launch_bounds__(256) void sub_dw_split_packed_kernel(uint16_t *out_hi, uint16_t *out_lo,
                                                                   const float *in, const int *oin,
-                                                                  const int *oout, int n, int Wd,
+                                                                  const int *oout, int n, int H_arg, int Wd,
                                                                   const uint16_t *w, const uint16_t *b) {
+    constexpr int NX = 2 * SUB_SEG + 1;
     const int Wo = (Wd + 1) / 2;
-    const int tau = blockIdx.x, c = threadIdx.x;
-    const int r = packed_owner(oout, n, tau);
-    const int oh = tau - oout[r], H = oin[r + 1] - oin[r];
-    const float *x = in + (long)oin[r] * Wd * SUB_CH + c;
+    const int tau = blockIdx.x, c = threadIdx.x, ow0 = blockIdx.y * SUB_SEG;
+    const int r = oout ? packed_owner(oout, n, tau) : 0;
+    const int oh = oout ? tau - oout[r] : tau, H = oout ? oin[r + 1] - oin[r] : H_arg;
+    const float *x = in + (long)(oout ? oin[r] : 0) * Wd * SUB_CH + c;
+    float v[3][NX];
+#pragma unroll
+    for (int kh = 0; kh < 3; kh++) {
+        const int ih = oh * 2 - 1 + kh;
+#pragma unroll
+        for (int j = 0; j < NX; j++) {
+            const int iw = 2 * ow0 - 1 + j;
+            v[kh][j] = ih >= 0 && ih < H && iw >= 0 && iw < Wd ? x[((long)ih * Wd + iw) * SUB_CH] : 0.0f;
+        }
+    }
     float k[9];
 #pragma unroll
     for (int j = 0; j < 9; j++) k[j] = bf2f(w[c * 9 + j]);
     const float bias = bf2f(b[c]);
-    for (int ow = 0; ow < Wo; ow++) {
+#pragma unroll
+    for (int j = 0; j < SUB_SEG; j++) {
+        if (ow0 + j >= Wo) break;
         float s = bias;
 #pragma unroll
-        for (int kh = 0; kh < 3; kh++) {
-            const int ih = oh * 2 - 1 + kh;
-            if (ih < 0 || ih >= H) continue;
+        for (int kh = 0; kh < 3; kh++)
 #pragma unroll
-            for (int kw = 0; kw < 3; kw++) {
-                const int iw = ow * 2 - 1 + kw;
-                if (iw < 0 || iw >= Wd) continue;
-                s += x[((long)ih * Wd + iw) * SUB_CH] * k[kh * 3 + kw];
-            }
-        }
+            for (int kw = 0; kw < 3; kw++) s += v[kh][2 * j + kw] * k[kh * 3 + kw];
         uint16_t hh, ll;
         split_bf16(s, hh, ll);
-        const long o = ((long)tau * Wo + ow) * SUB_CH + c;
+        const long o = ((long)tau * Wo + ow0 + j) * SUB_CH + c;
         out_hi[o] = hh;
         out_lo[o] = ll;
     }
@@ -642,16 +678,32 @@ extern "C" void ctk_sub_conv0_dw_packed(uint16_t *out_hi, uint16_t *out_lo, cons
                                         const uint16_t *w0, const uint16_t *b0, const uint16_t *wd,
                                         const uint16_t *bd, hipStream_t s) {
     if (rows2 <= 0 || n <= 0) return;
-    hipLaunchKernelGGL(sub_conv0_dw_packed_kernel, dim3(rows2), dim3(256), 0, s, out_hi, out_lo, mel, o1, o2,
-                       tmel, moff, n, w0, b0, wd, bd);
+    hipLaunchKernelGGL(sub_conv0_dw_packed_kernel, dim3(rows2, 32 / SUB_SEG), dim3(256), 0, s, out_hi, out_lo, mel, o1,
+                       o2, tmel, moff, n, 0, 0, w0, b0, wd, bd);
+}
+
+extern "C" void ctk_sub_conv0_dw(uint16_t *out_hi, uint16_t *out_lo, const float *mel, int T_mel, int stride,
+                                 const uint16_t *w0, const uint16_t *b0, const uint16_t *wd, const uint16_t *bd,
+                                 hipStream_t s) {
+    const int rows2 = ((T_mel + 1) / 2 + 1) / 2;
+    if (T_mel <= 0) return;
+    hipLaunchKernelGGL(sub_conv0_dw_packed_kernel, dim3(rows2, 32 / SUB_SEG), dim3(256), 0, s, out_hi, out_lo, mel,
+                       nullptr, nullptr, nullptr, nullptr, 1, T_mel, stride, w0, b0, wd, bd);
 }
 
 extern "C" void ctk_sub_dw_split_packed(uint16_t *out_hi, uint16_t *out_lo, const float *in, const int *oin,
                                         const int *oout, int n, int rows_out, int Wd, const uint16_t *w,
                                         const uint16_t *b, hipStream_t s) {
     if (rows_out <= 0 || n <= 0) return;
-    hipLaunchKernelGGL(sub_dw_split_packed_kernel, dim3(rows_out), dim3(256), 0, s, out_hi, out_lo, in, oin, oout,
-                       n, Wd, w, b);
+    hipLaunchKernelGGL(sub_dw_split_packed_kernel, dim3(rows_out, ((Wd + 1) / 2 + SUB_SEG - 1) / SUB_SEG), dim3(256), 0, s,
+                       out_hi, out_lo, in, oin, oout, n, 0, Wd, w, b);
+}
+
+extern "C" void ctk_sub_dw_split(uint16_t *out_hi, uint16_t *out_lo, const float *in, int H, int Wd, const uint16_t *w,
+                                 const uint16_t *b, hipStream_t s) {
+    if (H <= 0) return;
+    hipLaunchKernelGGL(sub_dw_split_packed_kernel, dim3((H + 1) / 2, ((Wd + 1) / 2 + SUB_SEG - 1) / SUB_SEG), dim3(256), 0,
+                       s, out_hi, out_lo, in, nullptr, nullptr, 1, H, Wd, w, b);
 }
 
 extern "C" void ctk_sub_flatten_split(uint16_t *hi, uint16_t *lo, const float *in, int T, hipStream_t s) {
