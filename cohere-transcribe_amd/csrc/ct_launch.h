@@ -70,7 +70,8 @@ void ctk_gemm(const CtGemm *g, hipStream_t s);
 #define CT_GEMM_GROUP 4
 void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s);
 /* Tests: 128 or 256 forces the pre-split kernels' tile, rows * 1000 + columns
- * a few-row tile (16016, 16032, 32032, 32064, 64128; 0: the cost model);
+ * a few-row tile (16016, 16032, 32032, 32064, 64128 and, of bf16 planes,
+ * 48128 (hi + lo only), 96128, 128128; 0: the cost model);
  * sizeof(CtGemm) for the tests' struct mirror. */
 void ctk_gemm_force_tile(int rows);
 int  ctk_gemm_sizeof(void);

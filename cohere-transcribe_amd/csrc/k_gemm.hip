@@ -1393,7 +1393,8 @@ __global__ __launch_bounds__(512) void gemm_split256_sp_kernel(CtGemm g, int n_m
 //
 // Measured (us; before -> now): fp32 activations 13 x 1280 x 1280 15 -> 6.6,
 // 101 x 1280 x 5120 161 -> 21, 376 x 5120 x 1280 49 -> 22; hi + lo planes
-// 101 x 1280 x 5120 114 -> 13, 1008 x 1280 x 5120 115 -> 46; hi alone
+// 101 x 1280 x 5120 114 -> 13, 1008 x 1280 x 5120 115 -> 40,
+// 2071 x 1280 x 5120 118 -> 66; hi alone
 // 101 x 1280 x 5120 76 -> 10 (13 MB of weights).
 // ---------------------------------------------------------------------------
 enum { A_F32 = 0, A_HILO = 1, A_HI = 2 };
@@ -1410,7 +1411,7 @@ struct RowsCfg {
     static constexpr int AHEAD = AM == A_F32 ? 2 : 1;
     static constexpr int LDS = NS * STAGE + 2 * NF * 2048;
     static constexpr int PL = AM == A_HILO ? NI_A / 2 : NI_A; // DMA instructions per A plane
-    static_assert(NI % P == 0 && PL % P == 0, "each DMA instruction j is of one operand for every producer");
+    static_assert(NI % P == 0, "every producer issues the same number of DMA instructions");
     static_assert((NS - 1) * PW <= 63, "vmcnt counts to 63");
     static_assert(LDS <= 160 * 1024 && WR * WC <= NW && NS > AHEAD, "LDS and wave budget");
 };
@@ -1426,10 +1427,10 @@ __device__ __forceinline__ void lds_dma16_saddr(const char *base, unsigned off, 
 
 // 16-byte slot of chunk c in LDS row R of NCH chunks.  Rows of 16 chunks or
 // more start on the same bank, so 16 rows take 16 slots; rows of 8 chunks
-// alternate between two halves of the banks.
+// alternate between two halves of the banks, rows of 4 between four quarters.
 template <int NCH>
 __device__ __forceinline__ int rswz(int R, int c) {
-    return c ^ (NCH >= 16 ? (R & 15) : ((R & 7) ^ ((R >> 3) & 1)));
+    return c ^ (NCH >= 16 ? (R & 15) : NCH == 8 ? ((R & 7) ^ ((R >> 3) & 1)) : (((R >> 1) ^ (R >> 2)) & 3));
 }
 
 // s_waitcnt vmcnt(y * PW) lgkmcnt(0) for a runtime y <= Y
@@ -1445,10 +1446,29 @@ __device__ __forceinline__ void wait_younger(int y) {
     __builtin_amdgcn_s_waitcnt((v & 15) | (7 << 4) | ((v >> 4) << 14));
 }
 
+// a pointer every lane holds alike, kept in scalar registers
+__device__ __forceinline__ const char *scalar_ptr(const char *p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (const char *)((uint64_t)hi << 32 | lo);
+}
+
+// DMA instruction J of a producer (pw of P): i = pw + P*J, an instruction of
+// A (hi), of its lo plane or of W
+template <class C, int J>
+__device__ __forceinline__ void dma_one(const char *pA, const char *pL, const char *pW, unsigned off, unsigned lds, int pw) {
+    constexpr int i0 = C::P * J, i1 = i0 + C::P;
+    const char *base;
+    if constexpr (i1 <= C::PL) base = pA;
+    else if constexpr (i0 >= C::NI_A) base = pW;
+    else if constexpr (i0 >= C::PL && i1 <= C::NI_A) base = pL;
+    else base = scalar_ptr(pw + i0 < C::PL ? pA : pw + i0 < C::NI_A ? pL : pW);
+    lds_dma16_saddr<i0 * 1024>(base, off, lds);
+}
 template <class C, int... J>
 __device__ __forceinline__ void dma_stage(const char *pA, const char *pL, const char *pW, const unsigned (&off)[C::PW],
-                                          unsigned lds, std::integer_sequence<int, J...>) {
-    (lds_dma16_saddr<C::P * J * 1024>(C::P * J >= C::NI_A ? pW : C::P * J >= C::PL ? pL : pA, off[J], lds), ...);
+                                          unsigned lds, int pw, std::integer_sequence<int, J...>) {
+    (dma_one<C, J>(pA, pL, pW, off[J], lds, pw), ...);
 }
 
 template <class C, bool GLU>
@@ -1477,7 +1497,7 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
 #pragma unroll
     for (int j = 0; j < PW; j++) {
         const int i = pw + P * j;
-        if (P * j < C::NI_A) {
+        if (i < C::NI_A) {
             constexpr int NCH = KS * EA / 16, RPI = 64 / NCH;
             const int R = (i % C::PL) * RPI + lane / NCH, ch = rswz<NCH>(R, lane % NCH);
             off[j] = (unsigned)((min(m0 + R, g.M - 1) - m0) * (int)g.lda * EA + ch * 16);   // rows >= M are never stored
@@ -1494,7 +1514,11 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(lds_ptr_t)smem) + pw * 1024;
     int slot = 0;
     auto issue = [&]() {
-        dma_stage<C>(pA, pL, pW, off, lds0 + slot, std::make_integer_sequence<int, PW>());
+        if constexpr (RB * CB >= 6) {
+            pA = scalar_ptr(pA); pL = scalar_ptr(pL); pW = scalar_ptr(pW);
+            slot = __builtin_amdgcn_readfirstlane(slot);
+        }
+        dma_stage<C>(pA, pL, pW, off, lds0 + slot, pw, std::make_integer_sequence<int, PW>());
         pA += KS * EA;
         if (AM == A_HILO) pL += KS * EA;
         pW += KS * 2;
@@ -1663,6 +1687,58 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
         if (++kt < nk) tail(1, f1, f0);
     }
     if (!comp) return;
+    // Rows that store to one place (plain rows, or a tile inside one dense or
+    // split segment): where, and whether the activation applies, once per tile
+    // instead of per element.
+    const int si = g.nseg > 0 ? c0 / g.seg_w : 0;
+    const bool inseg = g.nseg > 0 && (c0 + 16 * CO * C::WC - 1) / g.seg_w == si &&
+                       (g.seg[si].mode == CT_OUT_DENSE || g.seg[si].mode == CT_OUT_SPLIT);
+    if (!GLU && !g.row_mask && !g.row_len && (g.nseg == 0 || inseg)) {
+        const bool planes = inseg && g.seg[si].mode == CT_OUT_SPLIT;
+        const long ld = inseg ? g.seg[si].ld : g.ldy;
+        const int act = inseg && !planes ? CT_EPI_STORE : g.epi;
+        float *yf = inseg ? reinterpret_cast<float *>(g.seg[si].base) : g.Y;
+        uint16_t *yh = reinterpret_cast<uint16_t *>(yf);
+        uint16_t *yl = planes ? reinterpret_cast<uint16_t *>(g.seg[si].base_lo) : nullptr;
+        const int mb = m0 + wr * RB * 16 + kg * 4;
+#pragma unroll
+        for (int cb = 0; cb < CO; cb++) {
+            const int col = c0 + (wc * CO + cb) * 16 + r;
+            if (col >= g.N) continue;
+            const float bc = g.bias ? bf2f(bia[cb]) : 0.0f;
+            const long o0 = (long)mb * ld + (inseg ? col - si * g.seg_w : col);
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+                float v[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = acc[rb][cb][j] + bc;
+                if (fm) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = yres[rb][cb][j] + g.scale * v[j];
+                } else if (act == CT_EPI_SILU) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = v[j] * sigmoid_hw(v[j]);
+                } else if (act == CT_EPI_RELU) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = v[j] > 0.0f ? v[j] : 0.0f;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (mb + rb * 16 + j >= g.M) break;
+                    const long o = o0 + (rb * 16 + j) * ld;
+                    if (planes) {
+                        uint16_t h, l;
+                        split_bf16(v[j], h, l);
+                        yh[o] = h;
+                        if (yl) yl[o] = l;
+                    } else {
+                        yf[o] = v[j];
+                    }
+                }
+            }
+        }
+        return;
+    }
     // lane (r, kg) holds rows 4*kg + j, column r of each 16 x 16 block
 #pragma unroll
     for (int cb = 0; cb < CO; cb++) {
@@ -1733,16 +1809,23 @@ void launch_rows_cfg(const CtGemm &g, hipStream_t s, const CtGemmGroup *grp, int
     hipLaunchKernelGGL((gemm_rows_kernel<C, false>), dim3(blocks), dim3(64 * C::NW), 0, s, g, n_mt, nt);
 }
 
-// The few-row tiles, smallest first: rows, weight columns, whether the GLU
-// form exists (a wave needs an even number of column blocks), and the
-// measured us per 1000 of K of one workgroup per CU, for A_F32, A_HILO, A_HI.
-struct RowsTile { int tm, tn; bool glu; float us[3]; };
+// The few-row tiles: rows, weight columns, whether the GLU form exists (a wave
+// needs an even number of column blocks), and the measured us of one round of
+// workgroups per 1000 of K and besides, for A_F32, A_HILO, A_HI (0: no form).
+// The 48-, 96- and 128-row tiles are there for the rounds: 1280 columns of
+// 2071 rows are 330 tiles of 64 x 128, two rounds, and 220 of 96 x 128
+// (K = 5120, hi + lo: 95 and 66 us; 2700 rows in 128 x 128 86 for 97; 1008
+// rows in 48 x 128 40 for 46; GLU of 1008 rows in 96 x 128 20 for 27).
+struct RowsTile { int tm, tn; bool glu; float us[3], fix[3]; };
 constexpr RowsTile ROWS_TILES[] = {
-    {16, 16, false, {1.9f, 1.4f, 1.0f}},
-    {16, 32, true, {2.1f, 1.85f, 1.05f}},
-    {32, 32, false, {3.1f, 1.9f, 1.1f}},
-    {32, 64, true, {4.5f, 3.1f, 2.3f}},
-    {64, 128, true, {13.f, 8.4f, 5.6f}},
+    {16, 16, false, {1.9f, 1.4f, 1.0f}, {1.6f, 1.6f, 1.6f}},
+    {16, 32, true, {2.1f, 1.85f, 1.05f}, {1.6f, 1.6f, 1.6f}},
+    {32, 32, false, {3.1f, 1.9f, 1.1f}, {1.6f, 1.6f, 1.6f}},
+    {32, 64, true, {4.5f, 3.1f, 2.3f}, {1.6f, 1.6f, 1.6f}},
+    {64, 128, true, {13.f, 7.8f, 5.1f}, {5.5f, 6.0f, 6.0f}},
+    {48, 128, true, {0.f, 6.4f, 0.f}, {0.f, 7.7f, 0.f}},
+    {96, 128, true, {0.f, 11.3f, 7.8f}, {0.f, 7.7f, 6.0f}},
+    {128, 128, true, {0.f, 14.2f, 9.5f}, {0.f, 10.5f, 6.0f}},
 };
 constexpr int N_ROWS_TILES = sizeof ROWS_TILES / sizeof ROWS_TILES[0];
 
@@ -1757,8 +1840,20 @@ void launch_rows(int tile, const CtGemm &g, hipStream_t s, const CtGemmGroup *gr
         return launch_rows_cfg<RowsCfg<AM, 1, 1, 1, 2, 2, 6, 128, 4>>(g, s, grp, n);
     case 2: return launch_rows_cfg<RowsCfg<AM, 1, 1, 2, 2, 4, AM == A_F32 ? 12 : 8, 128, 4>>(g, s, grp, n);
     case 3: return launch_rows_cfg<RowsCfg<AM, 1, 2, 2, 2, 4, 8, 64, 4>>(g, s, grp, n);
-    default: return launch_rows_cfg<RowsCfg<AM, 2, 2, 2, 4, 0, 8, 64, AM == A_F32 ? 4 : 3>>(g, s, grp, n);
+    case 4: return launch_rows_cfg<RowsCfg<AM, 2, 2, 2, 4, 0, 8, 64, AM == A_F32 ? 4 : 3>>(g, s, grp, n);
+    case 5:
+        if constexpr (AM == A_HILO) return launch_rows_cfg<RowsCfg<AM, 3, 2, 1, 4, 4, 8, 64, 4>>(g, s, grp, n);
+        break;
+    case 6:
+        if constexpr (AM != A_F32)
+            return launch_rows_cfg<RowsCfg<AM, 3, 2, 2, 4, AM == A_HILO ? 0 : 4, 8, 64, 3>>(g, s, grp, n);
+        break;
+    case 7:
+        if constexpr (AM != A_F32) return launch_rows_cfg<RowsCfg<AM, 4, 4, 2, 2, 4, 8, 32, 4>>(g, s, grp, n);
+        break;
     }
+    fprintf(stderr, "ctk_gemm: few-row tile %d has no form for this input\n", tile);
+    exit(1);
 }
 
 __global__ void split_kernel(uint16_t *hi, uint16_t *lo, const float *x, long n) {
@@ -1958,8 +2053,8 @@ static int prefer_256(int M, int n_nt) {
 // 8.6 us more, hi + lo).  w: workgroups per CU.  Two small workgroups share a
 // CU at 1.55 times the cost each; the larger tiles run in rounds.  Where the
 // line falls (us, few-row against many-row): 1280 x 5120 hi + lo, 1500 rows
-// 50 against 115, 2700 rows 97 against 118; 3840 x 1280, 1008 rows 34 against
-// 38, 1500 rows 52 against 40.
+// 50 against 115, 2700 rows 86 against 118; 3840 x 1280, 1008 rows 30 against
+// 38, 1300 rows 40 against 39.
 static int rows_tile(const CtGemm *g, int am, int n = 1) {
     const bool glu = g->epi == CT_EPI_GLU;
     auto wgs = [&](int tm, int tc) {
@@ -1969,17 +2064,17 @@ static int rows_tile(const CtGemm *g, int am, int n = 1) {
         return t / cu_count();
     };
     // every DMA address is a base and a 32-bit offset within the tile's rows
-    const long wspan = (long)(glu ? g->glu_half + 256 : 256) * g->K * 2, aspan = 64L * g->lda * 4;
+    const long wspan = (long)(glu ? g->glu_half + 256 : 256) * g->K * 2, aspan = 128L * g->lda * 4;
     if (g->K % 128 || wspan >= 1L << 31 || aspan >= 1L << 31) return -1;
     const double k = g->K / 1000.0;
     int best = -1;
     double bt = 0;
     for (int i = 0; i < N_ROWS_TILES; i++) {
         const RowsTile &t = ROWS_TILES[i];
-        if (glu && !t.glu) continue;
+        if ((glu && !t.glu) || t.us[am] == 0) continue;
         const double w = wgs(t.tm, glu ? t.tn / 2 : t.tn);
-        const double us = t.tm == 64 ? ceil(w) * (k * t.us[am] + 5.5)
-                                     : k * t.us[am] * (w <= 1 ? 1 : 1.55 * w) + 1.6 * (w <= 1 ? 1 : w);
+        const double us = t.tm >= 48 ? ceil(w) * (k * t.us[am] + t.fix[am])
+                                     : k * t.us[am] * (w <= 1 ? 1 : 1.55 * w) + t.fix[am] * (w <= 1 ? 1 : w);
         if (g_force_tile ? g_force_tile == t.tm * 1000 + t.tn : best < 0 || us < bt) { best = i; bt = us; }
     }
     if (g_force_tile) return best;
