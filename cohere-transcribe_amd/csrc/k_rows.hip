@@ -235,27 +235,48 @@ __device__ __forceinline__ void better(float &bv, int &bi, float v, int i) {
     if (v > bv || (v == bv && i < bi)) { bv = v; bi = i; }
 }
 
-__global__ __launch_bounds__(256) void argmax_kernel(int *out, const float *logits, int n,
-                                                     const int *active) {
+// A workgroup of 1024 threads per row; rows of whole, aligned float4 are read
+// four loads deep.  48 rows of 16384: 22 -> 6 us (256 threads, a load at a time).
+constexpr int AM_NT = 1024;
+template <bool VEC>
+__global__ __launch_bounds__(AM_NT) void argmax_kernel(int *out, const float *logits, int n,
+                                                       const int *active) {
     const int r = blockIdx.x;
     if (active && !active[r]) return;
     const float *x = logits + (long)r * n;
     float bv = -INFINITY;
     int bi = INT_MAX;
-    for (int i = threadIdx.x; i < n; i += 256) better(bv, bi, x[i], i);
+    int i0 = 0;
+    if (VEC) {
+        const float4 *x4 = reinterpret_cast<const float4 *>(x);
+        for (; i0 + 16 * AM_NT <= n; i0 += 16 * AM_NT) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = x4[i0 / 4 + u * AM_NT + threadIdx.x];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int i = i0 + 4 * (u * AM_NT + threadIdx.x);
+                better(bv, bi, v[u].x, i);
+                better(bv, bi, v[u].y, i + 1);
+                better(bv, bi, v[u].z, i + 2);
+                better(bv, bi, v[u].w, i + 3);
+            }
+        }
+    }
+    for (int i = i0 + threadIdx.x; i < n; i += AM_NT) better(bv, bi, x[i], i);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const float ov = __shfl_xor(bv, o, 64);
         const int oi = __shfl_xor(bi, o, 64);
         better(bv, bi, ov, oi);
     }
-    __shared__ float sv[4];
-    __shared__ int si[4];
+    __shared__ float sv[AM_NT / 64];
+    __shared__ int si[AM_NT / 64];
     const int wv = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) { sv[wv] = bv; si[wv] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int k = 1; k < 4; k++) better(bv, bi, sv[k], si[k]);
+        for (int k = 1; k < AM_NT / 64; k++) better(bv, bi, sv[k], si[k]);
         out[r] = (x[0] != x[0] || bi == INT_MAX) ? 0 : bi;
     }
 }
@@ -531,7 +552,10 @@ extern "C" void ctk_embed_fold(float *h, float *lnstat, uint16_t *frag, const in
 extern "C" void ctk_argmax(int *out, const float *logits, int R, int n, const int *active,
                            hipStream_t s) {
     if (R <= 0) return;
-    hipLaunchKernelGGL(argmax_kernel, dim3(R), dim3(256), 0, s, out, logits, n, active);
+    if (n % 4 == 0 && ((uintptr_t)logits & 15) == 0)
+        hipLaunchKernelGGL(argmax_kernel<true>, dim3(R), dim3(AM_NT), 0, s, out, logits, n, active);
+    else
+        hipLaunchKernelGGL(argmax_kernel<false>, dim3(R), dim3(AM_NT), 0, s, out, logits, n, active);
 }
 
 extern "C" void ctk_add(float *dst, const float *src, long n, hipStream_t s) {
