@@ -150,6 +150,11 @@ struct HipbEngine {
     int bench_gemm_M;    /* rows seeded by hipb_bench_encoder_gemm */
     /* log-mel front-end */
     CtMelTables mel_tab;
+    /* hipb_mel's device buffers, kept between calls (at most CT_MEL_WS_MAX
+     * bytes), one call at a time under mel_mu */
+    pthread_mutex_t mel_mu;
+    void *mel_ws;
+    size_t mel_ws_bytes;
     float *d_hann, *d_twr, *d_twi, *d_fb;
     int *d_fb_lo, *d_fb_hi;
     float *epcm;
@@ -451,6 +456,7 @@ HipbEngine *hipb_create(const HipbConfig *cfg, const Weights *W) {
     e->free_head = 0;
     e->free_tail = R;
     pthread_mutex_init(&e->mu, NULL);
+    pthread_mutex_init(&e->mel_mu, NULL);
     pthread_cond_init(&e->cv, NULL);
     const char *eg = getenv("HIPB_EAGER");
     e->eager = eg && eg[0] == '1';
@@ -488,7 +494,7 @@ void hipb_destroy(HipbEngine *e) {
                     e->e_blk_seq, e->e_blk_q0, e->e_rowoff, e->d_hann, e->d_twr, e->d_twi, e->d_fb,
                     e->d_fb_lo, e->d_fb_hi, e->epcm, e->e_clips, e->e_frame_clip,
                     e->eln_h, e->eln_l, e->emid_h, e->emid_l, e->eo_h, e->eo_l, e->edw_h, e->edw_l,
-                    e->floor_sink};
+                    e->floor_sink, e->mel_ws};
     for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
         if (ptrs[i]) ECHK(hipFree(ptrs[i]));
     for (int r = 0; r < e->n_req; r++) {
@@ -499,6 +505,7 @@ void hipb_destroy(HipbEngine *e) {
     free(e->free_ent);
     free(e->ent_owner);
     pthread_mutex_destroy(&e->mu);
+    pthread_mutex_destroy(&e->mel_mu);
     pthread_cond_destroy(&e->cv);
     ECHK(hipHostFree(e->h_tmp));
     ECHK(hipHostFree(e->h_meta));
@@ -1836,12 +1843,28 @@ void hipb_bench_encoder_gemm(HipbEngine *e, int M) {
                        sp ? NULL : e->emid_l);
 }
 
+/* device bytes hipb_mel keeps: a clip of about 10 minutes */
+#define CT_MEL_WS_MAX ((size_t)64 << 20)
+
 void hipb_mel(HipbEngine *e, const float *pcm, int n_samples, float *mel_out) {
     if (n_samples < HOP_LEN) CT_FATAL("hipb_mel: clip shorter than one hop (160 samples)");
     const int T = 1 + n_samples / HOP_LEN;
-    float *dp = dmalloc((size_t)n_samples * 4), *dm = dmalloc((size_t)N_MELS * T * 4);
-    CtMelClip *dc = dmalloc(sizeof(CtMelClip));
-    int *fc = dmalloc((size_t)T * sizeof(int));
+    /* one allocation: clip, frame table, spectrogram, samples */
+    const size_t o_fc = 256, o_mel = o_fc + ((size_t)T * sizeof(int) + 255) / 256 * 256;
+    const size_t o_pcm = o_mel + (size_t)N_MELS * T * 4, need = o_pcm + (size_t)n_samples * 4;
+    pthread_mutex_lock(&e->mel_mu);
+    char *ws = e->mel_ws;
+    if (need > e->mel_ws_bytes) {
+        ws = dmalloc(need);
+        if (need <= CT_MEL_WS_MAX) {
+            if (e->mel_ws) ECHK(hipFree(e->mel_ws));
+            e->mel_ws = ws;
+            e->mel_ws_bytes = need;
+        }
+    }
+    float *dp = (float *)(ws + o_pcm), *dm = (float *)(ws + o_mel);
+    CtMelClip *dc = (CtMelClip *)ws;
+    int *fc = (int *)(ws + o_fc);
     const CtMelClip c = {dp, n_samples, 0, T, 0};
     ECHK(hipMemcpyAsync(dp, pcm, (size_t)n_samples * 4, hipMemcpyHostToDevice, e->s));
     ECHK(hipMemcpyAsync(dc, &c, sizeof c, hipMemcpyHostToDevice, e->s));
@@ -1849,5 +1872,6 @@ void hipb_mel(HipbEngine *e, const float *pcm, int n_samples, float *mel_out) {
     ctk_mel(dm, dc, 1, fc, T, &e->mel_tab, e->s);
     ECHK(hipMemcpyAsync(mel_out, dm, (size_t)N_MELS * T * 4, hipMemcpyDeviceToHost, e->s));
     ECHK(hipStreamSynchronize(e->s));
-    ECHK(hipFree(dp)); ECHK(hipFree(dm)); ECHK(hipFree(dc)); ECHK(hipFree(fc));
+    if (ws != e->mel_ws) ECHK(hipFree(ws));
+    pthread_mutex_unlock(&e->mel_mu);
 }

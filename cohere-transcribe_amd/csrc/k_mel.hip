@@ -4,7 +4,7 @@
 // (200 each side), pre-emphasised (x[i] - 0.97 x[i-1]) signal, Hann window,
 // 512-point FFT, power spectrum (257 bins), 128 Slaney mel filters,
 // log(x + 2^-24).  Then each mel bin is normalised over the clip's frames
-// with mean and var/(T-1).  One workgroup transforms one frame in LDS
+// with mean and var/(T-1).  One wavefront transforms one frame in LDS
 // (radix-2, twiddles from a host table); a second kernel normalises rows.
 #include "ct_dev.h"
 #include "ct_launch.h"
@@ -13,21 +13,38 @@
 namespace {
 
 constexpr int NF = N_FFT;   // 512
+constexpr int FPW = 4;      // frames of a workgroup, one per wavefront
 
-__global__ __launch_bounds__(256) void mel_frames_kernel(float *mel,
+// Orders one wavefront's LDS accesses: the hardware keeps them in issue order,
+// so only the compiler has to be held.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A wavefront transforms one frame alone, four butterflies a lane and stage,
+// so no stage waits for other wavefronts (one frame on four wavefronts spent
+// its time at 18 barriers): 2001 frames 16.5 -> 15.1 us, 16503 89 -> 63.
+__global__ __launch_bounds__(64 * FPW) void mel_frames_kernel(float *mel,
                                                          const CtMelClip *clips, const int *frame_clip,
                                                          const float *hann, const float *twr,
                                                          const float *twi, const float *fb,
-                                                         const int *fb_lo, const int *fb_hi) {
-    __shared__ float re[NF], im[NF], ps[N_BINS];
-    const int f = blockIdx.x;
+                                                         const int *fb_lo, const int *fb_hi, int n_frames) {
+    __shared__ float s_re[FPW][NF], s_im[FPW][NF], s_wr[NF / 2], s_wi[NF / 2];
+    for (int i = threadIdx.x; i < NF / 2; i += 64 * FPW) { s_wr[i] = twr[i]; s_wi[i] = twi[i]; }
+    __syncthreads();
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int f = blockIdx.x * FPW + w;
+    if (f >= n_frames) return;
+    float *re = s_re[w], *im = s_im[w];
     const CtMelClip c = clips[frame_clip[f]];
     const int t = f - c.frame0;
-    const int tid = threadIdx.x;
     const int off = t * HOP_LEN;
     const int pad = WIN_LEN / 2;
     // load windowed, pre-emphasised samples in bit-reversed order
-    for (int j = tid; j < NF; j += 256) {
+#pragma unroll
+    for (int j0 = 0; j0 < NF; j0 += 64) {
+        const int j = j0 + lane;
         float v = 0.0f;
         if (j < WIN_LEN) {
             const int a = off + j - pad;              // index into the clip
@@ -39,42 +56,86 @@ __global__ __launch_bounds__(256) void mel_frames_kernel(float *mel,
         re[r] = v;
         im[r] = 0.0f;
     }
-    __syncthreads();
+    wave_lds_fence();
     for (int half = 1; half < NF; half <<= 1) {
-        const int k = tid;                         // 256 butterflies per stage
-        const int grp = k / half, pos = k % half;
-        const int i0 = grp * 2 * half + pos, i1 = i0 + half;
-        const int tw = pos * (NF / (2 * half));
-        const float wr = twr[tw], wi = twi[tw];
-        const float vr = re[i1] * wr - im[i1] * wi;
-        const float vi = re[i1] * wi + im[i1] * wr;
-        const float ur = re[i0], ui = im[i0];
-        __syncthreads();
-        re[i0] = ur + vr; im[i0] = ui + vi;
-        re[i1] = ur - vr; im[i1] = ui - vi;
-        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NF / 128; u++) {           // 256 butterflies per stage
+            const int k = lane + 64 * u, pos = k & (half - 1);
+            const int i0 = 2 * k - pos, i1 = i0 + half;
+            const int tw = pos * (NF / (2 * half));
+            const float wr = s_wr[tw], wi = s_wi[tw];
+            const float vr = re[i1] * wr - im[i1] * wi;
+            const float vi = re[i1] * wi + im[i1] * wr;
+            const float ur = re[i0], ui = im[i0];
+            re[i0] = ur + vr; im[i0] = ui + vi;
+            re[i1] = ur - vr; im[i1] = ui - vi;
+        }
+        wave_lds_fence();
     }
-    for (int i = tid; i < N_BINS; i += 256) ps[i] = re[i] * re[i] + im[i] * im[i];
-    __syncthreads();
-    if (tid < N_MELS) {
+    // the power spectrum over the real parts (each lane reads only what it writes)
+    for (int i = lane; i < N_BINS; i += 64) re[i] = re[i] * re[i] + im[i] * im[i];
+    wave_lds_fence();
+    for (int m = lane; m < N_MELS; m += 64) {
         float acc = 0.0f;
-        for (int i = fb_lo[tid]; i < fb_hi[tid]; i++) acc += fb[tid * N_BINS + i] * ps[i];
-        mel[c.mel0 + (long)tid * c.T + t] = logf(acc + 5.9604644775390625e-8f);
+        const int lo = fb_lo[m], hi = fb_hi[m];
+        const float *wm = fb + m * N_BINS;
+        for (int i = lo; i < hi; i += 8) {             // eight weights in flight
+            float wt[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) wt[u] = i + u < hi ? wm[i + u] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (i + u < hi) acc += wt[u] * re[i + u];
+        }
+        mel[c.mel0 + (long)m * c.T + t] = logf(acc + 5.9604644775390625e-8f);
     }
 }
 
-__global__ __launch_bounds__(64) void mel_norm_kernel(float *mel, const CtMelClip *clips) {
+// One row of a clip's spectrogram per workgroup; up to MN_NT * MN_PER frames
+// stay in registers between the passes (a clip of 40 s), further ones are read
+// again.  The sums over threads are in 64 bits.  20 s on one wavefront 16.4 us,
+// here 4.3.
+constexpr int MN_NT = 512, MN_PER = 8;
+__device__ __forceinline__ double block_sum(double v, double *red) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = red[0];
+#pragma unroll
+    for (int i = 1; i < MN_NT / 64; i++) s += red[i];
+    return s;
+}
+__global__ __launch_bounds__(MN_NT) void mel_norm_kernel(float *mel, const CtMelClip *clips) {
+    __shared__ double red[2][MN_NT / 64];
     const CtMelClip c = clips[blockIdx.y];
-    const int m = blockIdx.x, lane = threadIdx.x;
+    const int m = blockIdx.x, tid = threadIdx.x;
     float *row = mel + c.mel0 + (long)m * c.T;
+    float v[MN_PER];
     float s = 0.0f;
-    for (int t = lane; t < c.T; t += 64) s += row[t];
-    const float mu = wave_sum(s) / (float)c.T;
+#pragma unroll
+    for (int i = 0; i < MN_PER; i++) {
+        const int t = tid + MN_NT * i;
+        v[i] = t < c.T ? row[t] : 0.0f;
+        s += v[i];
+    }
+    for (int t = tid + MN_NT * MN_PER; t < c.T; t += MN_NT) s += row[t];
+    const float mu = (float)(block_sum(s, red[0]) / c.T);
     float q = 0.0f;
-    for (int t = lane; t < c.T; t += 64) { const float d = row[t] - mu; q += d * d; }
-    const float var = wave_sum(q) / (float)(c.T - 1);
+#pragma unroll
+    for (int i = 0; i < MN_PER; i++) {
+        const float d = tid + MN_NT * i < c.T ? v[i] - mu : 0.0f;
+        q += d * d;
+    }
+    for (int t = tid + MN_NT * MN_PER; t < c.T; t += MN_NT) { const float d = row[t] - mu; q += d * d; }
+    const float var = (float)(block_sum(q, red[1]) / (c.T - 1));
     const float r = 1.0f / sqrtf(var + 1e-5f);
-    for (int t = lane; t < c.T; t += 64) row[t] = (row[t] - mu) * r;
+#pragma unroll
+    for (int i = 0; i < MN_PER; i++) {
+        const int t = tid + MN_NT * i;
+        if (t < c.T) row[t] = (v[i] - mu) * r;
+    }
+    for (int t = tid + MN_NT * MN_PER; t < c.T; t += MN_NT) row[t] = (row[t] - mu) * r;
 }
 
 }  // namespace
@@ -82,7 +143,7 @@ __global__ __launch_bounds__(64) void mel_norm_kernel(float *mel, const CtMelCli
 extern "C" void ctk_mel(float *mel, const CtMelClip *clips, int n_clips,
                         const int *frame_clip, int n_frames, const CtMelTables *tab, hipStream_t s) {
     if (n_frames <= 0) return;
-    hipLaunchKernelGGL(mel_frames_kernel, dim3(n_frames), dim3(256), 0, s, mel, clips, frame_clip,
-                       tab->hann, tab->twr, tab->twi, tab->fb, tab->fb_lo, tab->fb_hi);
-    hipLaunchKernelGGL(mel_norm_kernel, dim3(N_MELS, n_clips), dim3(64), 0, s, mel, clips);
+    hipLaunchKernelGGL(mel_frames_kernel, dim3((n_frames + FPW - 1) / FPW), dim3(64 * FPW), 0, s, mel, clips, frame_clip,
+                       tab->hann, tab->twr, tab->twi, tab->fb, tab->fb_lo, tab->fb_hi, n_frames);
+    hipLaunchKernelGGL(mel_norm_kernel, dim3(N_MELS, n_clips), dim3(MN_NT), 0, s, mel, clips);
 }

@@ -1,0 +1,66 @@
+"""GPU checks of the log-mel front-end's and the argmax's launch shapes: clips of
+few frames (a workgroup's last wavefronts without a frame), of a whole number of
+workgroups, and longer than the rows kept in registers (4096 frames); rows of
+logits of whole float4 and not, with ties, NaN and infinities.
+
+The spectrogram is held to the oracle's within the tolerance that
+test_gpu_engine.py derives for it (twiddle recurrence against exact twiddles).
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import ctbind as cb
+import oracle_bind as ob
+from test_gpu_gemv import Dev
+
+pytestmark = pytest.mark.gpu
+
+
+def test_mel_lengths(hip, kernel_model):
+    hip.backend_weights_upload_blob(kernel_model.data_ptr, kernel_model.data_bytes)
+    eng = cb.Engine(kernel_model, slots=1, max_requests=2, max_frames=40, kv_bf16=True)
+    try:
+        # short after long: the kept buffers are longer than the clip
+        for n in (160, 3 * 160, 4 * 160 + 1, 4097 * 160, 1000):
+            x = cb.synth_audio(n, n)
+            print(f"case: mel n={n}", flush=True)
+            got, ref = eng.mel(x), ob.compute_mel(x)
+            assert got.shape == ref.shape
+            assert np.abs(got - ref).max() < 2e-3, n
+            assert np.array_equal(got, eng.mel(x))
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1000, 4096, 16384, 16385, 16388, 40000])
+def test_argmax_rows(hip, n):
+    L = C.CDLL(cb.HIP_LIB)
+    L.ctk_argmax.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
+    dev = Dev(hip)
+    rng = np.random.default_rng(n)
+    R = 9
+    x = rng.integers(-50, 50, (R, n)).astype(np.float32)     # ties: the lowest index wins
+    x[1] = -np.inf
+    x[2, n // 2] = np.nan                                    # NaN never wins ..
+    x[3, 0] = np.nan                                         # .. but stays the answer at index 0
+    x[4, n - 1] = np.inf
+    x[5] = np.nan
+    x[6] = np.finfo(np.float32).min
+    want = []
+    for row in x:
+        best = 0
+        if row[0] == row[0]:
+            clean = np.where(np.isnan(row), -np.inf, row)
+            best = int(np.argmax(clean))
+        want.append(best)
+    act = np.ones(R, np.int32)
+    act[8] = 0
+    po, px, pa = dev.put(np.full(R, -5, np.int32)), dev.put(x), dev.put(act)
+    dev.ev.sync()
+    print(f"case: argmax n={n}", flush=True)
+    L.ctk_argmax(po, px, R, n, pa, None)
+    got = dev.get(po, np.int32, R)
+    assert got[8] == -5
+    assert np.array_equal(got[:8], want[:8])
