@@ -1375,7 +1375,7 @@ __global__ __launch_bounds__(512) void gemm_split256_sp_kernel(CtGemm g, int n_m
 
 // ---------------------------------------------------------------------------
 // Few-row encoder GEMM: small tiles, so that the rows of one clip or a few
-// (13 to about 2000) fill the chip.  With the 128-row tiles a 1280-column
+// (13 to about 3000) fill the chip.  With the 128-row tiles a 1280-column
 // product of an 8 s clip (101 rows) ran on 5 or 10 CUs and took the time of
 // one tile's K loop.  A row's K loop stays one chain of MFMAs in the same
 // order (K-steps, hi then lo), so the bits are those of the other kernels;
@@ -1389,7 +1389,7 @@ __global__ __launch_bounds__(512) void gemm_split256_sp_kernel(CtGemm g, int n_m
 // scalar base and a constant lane offset, and, for fp32 activations, split
 // each 16 x 32 fragment into hi and lo once per workgroup, two stages ahead.
 // One barrier per stage.  LDS rows are swizzled for both the DMA (1 KB runs)
-// and the fragment reads.  In the 64 x 128 tile every wave does both.
+// and the fragment reads.  In the 64- and 96-row tiles waves have both roles.
 //
 // Measured (us; before -> now): fp32 activations 13 x 1280 x 1280 15 -> 6.6,
 // 101 x 1280 x 5120 161 -> 21, 376 x 5120 x 1280 49 -> 22; hi + lo planes
