@@ -7,6 +7,7 @@ The spectrogram is held to the oracle's within the tolerance that
 test_gpu_engine.py derives for it (twiddle recurrence against exact twiddles).
 """
 import ctypes as C
+import hashlib
 
 import numpy as np
 import pytest
@@ -30,6 +31,31 @@ def test_mel_lengths(hip, kernel_model):
             assert got.shape == ref.shape
             assert np.abs(got - ref).max() < 2e-3, n
             assert np.array_equal(got, eng.mel(x))
+    finally:
+        eng.close()
+
+
+# samples: SHA-256 (first 16 digits) of the spectrogram whose rows are summed by
+# 64 lanes in fp32, each lane its own frames in turn and every square fused
+# into its sum, the lanes by wave_sum
+MEL_BITS = {
+    160: "b4e64e235ea18f25", 641: "247ea271ee4d5e36", 1000: "9683ffde0b0f3c68", 8000: "ae1c442037cc9fd9",
+    16000: "5de6fea4e623cd40", 41000: "2260df0d47755b46", 163000: "3d027f43b70a4d6e", 164000: "4c6cf605bca0fe3d",
+    320000: "7b33943304d1e715", 480000: "34f949f46aa91410", 655200: "04785f2544b22847", 655520: "8a2161bebd3f6645",
+}
+
+
+def test_mel_bits(hip, kernel_model):
+    """The spectrogram's bits do not depend on how the launches are split: 48
+    layers follow, and where their FFN rounds activations to bf16 a changed last
+    bit grows to 3e-3 of the encoder's output."""
+    hip.backend_weights_upload_blob(kernel_model.data_ptr, kernel_model.data_bytes)
+    eng = cb.Engine(kernel_model, slots=1, max_requests=2, max_frames=40, kv_bf16=True)
+    try:
+        for n, want in MEL_BITS.items():
+            x = (np.random.default_rng(n).integers(-8192, 8193, n) / np.float32(32768)).astype(np.float32)
+            print(f"case: mel bits n={n}", flush=True)
+            assert hashlib.sha256(eng.mel(x).tobytes()).hexdigest()[:16] == want, n
     finally:
         eng.close()
 
