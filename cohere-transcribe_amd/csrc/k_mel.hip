@@ -4,8 +4,9 @@
 // (200 each side), pre-emphasised (x[i] - 0.97 x[i-1]) signal, Hann window,
 // 512-point FFT, power spectrum (257 bins), 128 Slaney mel filters,
 // log(x + 2^-24).  Then each mel bin is normalised over the clip's frames
-// with mean and var/(T-1).  One wavefront transforms one frame in LDS
-// (radix-2, twiddles from a host table); a second kernel normalises rows.
+// with mean and var/(T-1).  One wavefront, or with few frames four, transform
+// one frame in LDS (radix-2, twiddles from a host table); a second kernel
+// normalises rows.
 #include "ct_dev.h"
 #include "ct_launch.h"
 #include "../../include/model_types.h"
@@ -13,7 +14,6 @@
 namespace {
 
 constexpr int NF = N_FFT;   // 512
-constexpr int FPW = 4;      // frames of a workgroup, one per wavefront
 
 // Orders one wavefront's LDS accesses: the hardware keeps them in issue order,
 // so only the compiler has to be held.
@@ -22,19 +22,32 @@ __device__ __forceinline__ void wave_lds_fence() {
     asm volatile("" ::: "memory");
 }
 
-// A wavefront transforms one frame alone, four butterflies a lane and stage,
-// so no stage waits for other wavefronts (one frame on four wavefronts spent
-// its time at 18 barriers): 2001 frames 16.5 -> 15.1 us, 16503 89 -> 63.
-__global__ __launch_bounds__(64 * FPW) void mel_frames_kernel(float *mel,
+// A workgroup of four wavefronts takes WPF of them per frame.  With many frames
+// each wavefront transforms one alone (WPF 1): four butterflies a lane and
+// stage, no barriers.  With few, nothing hides that chain, and the frame is
+// split over the workgroup (WPF 4): one butterfly a lane and a barrier per
+// stage.  Both do the same arithmetic per element.  us, WPF 1 and 4: 51 frames
+// 11.3 and 6.3, 301 11.9 and 6.7, 1019 12.5 and 9.7, 2001 14.2 and 14.4, 3001
+// 18.3 and 18.4, 4096 20.9 and 22.9, 6251 29 and 32; 16503 with WPF 1 63 (89
+// with twiddles from memory and two barriers a stage).
+constexpr int MEL_FEW_FRAMES = 2048;
+template <int WPF>
+__global__ __launch_bounds__(256) void mel_frames_kernel(float *mel,
                                                          const CtMelClip *clips, const int *frame_clip,
                                                          const float *hann, const float *twr,
                                                          const float *twi, const float *fb,
                                                          const int *fb_lo, const int *fb_hi, int n_frames) {
+    constexpr int FPW = 4 / WPF, LANES = 64 * WPF;
     __shared__ float s_re[FPW][NF], s_im[FPW][NF], s_wr[NF / 2], s_wi[NF / 2];
-    for (int i = threadIdx.x; i < NF / 2; i += 64 * FPW) { s_wr[i] = twr[i]; s_wi[i] = twi[i]; }
-    __syncthreads();
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int w = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     const int f = blockIdx.x * FPW + w;
+    s_wr[threadIdx.x] = twr[threadIdx.x];
+    s_wi[threadIdx.x] = twi[threadIdx.x];
+    auto frame_sync = [] {
+        if (WPF == 1) wave_lds_fence();
+        else __syncthreads();
+    };
+    if (WPF == 1) __syncthreads();
     if (f >= n_frames) return;
     float *re = s_re[w], *im = s_im[w];
     const CtMelClip c = clips[frame_clip[f]];
@@ -43,7 +56,7 @@ __global__ __launch_bounds__(64 * FPW) void mel_frames_kernel(float *mel,
     const int pad = WIN_LEN / 2;
     // load windowed, pre-emphasised samples in bit-reversed order
 #pragma unroll
-    for (int j0 = 0; j0 < NF; j0 += 64) {
+    for (int j0 = 0; j0 < NF; j0 += LANES) {
         const int j = j0 + lane;
         float v = 0.0f;
         if (j < WIN_LEN) {
@@ -56,11 +69,11 @@ __global__ __launch_bounds__(64 * FPW) void mel_frames_kernel(float *mel,
         re[r] = v;
         im[r] = 0.0f;
     }
-    wave_lds_fence();
+    frame_sync();
     for (int half = 1; half < NF; half <<= 1) {
 #pragma unroll
-        for (int u = 0; u < NF / 128; u++) {           // 256 butterflies per stage
-            const int k = lane + 64 * u, pos = k & (half - 1);
+        for (int u = 0; u < NF / 2 / LANES; u++) {     // 256 butterflies per stage
+            const int k = lane + LANES * u, pos = k & (half - 1);
             const int i0 = 2 * k - pos, i1 = i0 + half;
             const int tw = pos * (NF / (2 * half));
             const float wr = s_wr[tw], wi = s_wi[tw];
@@ -70,12 +83,12 @@ __global__ __launch_bounds__(64 * FPW) void mel_frames_kernel(float *mel,
             re[i0] = ur + vr; im[i0] = ui + vi;
             re[i1] = ur - vr; im[i1] = ui - vi;
         }
-        wave_lds_fence();
+        frame_sync();
     }
     // the power spectrum over the real parts (each lane reads only what it writes)
-    for (int i = lane; i < N_BINS; i += 64) re[i] = re[i] * re[i] + im[i] * im[i];
-    wave_lds_fence();
-    for (int m = lane; m < N_MELS; m += 64) {
+    for (int i = lane; i < N_BINS; i += LANES) re[i] = re[i] * re[i] + im[i] * im[i];
+    frame_sync();
+    for (int m = lane; m < N_MELS; m += LANES) {
         float acc = 0.0f;
         const int lo = fb_lo[m], hi = fb_hi[m];
         const float *wm = fb + m * N_BINS;
@@ -165,7 +178,11 @@ __global__ __launch_bounds__(64) void mel_norm_kernel(float *mel, const CtMelCli
 extern "C" void ctk_mel(float *mel, const CtMelClip *clips, int n_clips,
                         const int *frame_clip, int n_frames, const CtMelTables *tab, hipStream_t s) {
     if (n_frames <= 0) return;
-    hipLaunchKernelGGL(mel_frames_kernel, dim3((n_frames + FPW - 1) / FPW), dim3(64 * FPW), 0, s, mel, clips, frame_clip,
-                       tab->hann, tab->twr, tab->twi, tab->fb, tab->fb_lo, tab->fb_hi, n_frames);
+    if (n_frames <= MEL_FEW_FRAMES)
+        hipLaunchKernelGGL(mel_frames_kernel<4>, dim3(n_frames), dim3(256), 0, s, mel, clips, frame_clip, tab->hann,
+                           tab->twr, tab->twi, tab->fb, tab->fb_lo, tab->fb_hi, n_frames);
+    else
+        hipLaunchKernelGGL(mel_frames_kernel<1>, dim3((n_frames + 3) / 4), dim3(256), 0, s, mel, clips, frame_clip,
+                           tab->hann, tab->twr, tab->twi, tab->fb, tab->fb_lo, tab->fb_hi, n_frames);
     hipLaunchKernelGGL(mel_norm_kernel, dim3(N_MELS, n_clips), dim3(64), 0, s, mel, clips);
 }

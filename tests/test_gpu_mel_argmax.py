@@ -37,8 +37,10 @@ def test_mel_lengths(hip, kernel_model):
 
 # samples: SHA-256 (first 16 digits) of the spectrogram whose rows are summed by
 # 64 lanes in fp32, each lane its own frames in turn and every square fused
-# into its sum, the lanes by wave_sum
+# into its sum, the lanes by wave_sum.  Frames a clip: few (four wavefronts a
+# frame) up to 2048 = 327520 samples, one wavefront a frame from 2049 on.
 MEL_BITS = {
+    327520: "605bf024add393b3", 327680: "c81eeea31b284681",
     160: "b4e64e235ea18f25", 641: "247ea271ee4d5e36", 1000: "9683ffde0b0f3c68", 8000: "ae1c442037cc9fd9",
     16000: "5de6fea4e623cd40", 41000: "2260df0d47755b46", 163000: "3d027f43b70a4d6e", 164000: "4c6cf605bca0fe3d",
     320000: "7b33943304d1e715", 480000: "34f949f46aa91410", 655200: "04785f2544b22847", 655520: "8a2161bebd3f6645",
