@@ -150,8 +150,8 @@ struct HipbEngine {
     int bench_gemm_M;    /* rows seeded by hipb_bench_encoder_gemm */
     /* log-mel front-end */
     CtMelTables mel_tab;
-    /* hipb_mel's device buffers, kept between calls (at most CT_MEL_WS_MAX
-     * bytes), one call at a time under mel_mu */
+    /* a device buffer of hipb_mel kept for its next call (at most
+     * CT_MEL_WS_MAX bytes); mel_mu covers taking it and giving it back */
     pthread_mutex_t mel_mu;
     void *mel_ws;
     size_t mel_ws_bytes;
@@ -1843,25 +1843,52 @@ void hipb_bench_encoder_gemm(HipbEngine *e, int M) {
                        sp ? NULL : e->emid_l);
 }
 
-/* device bytes hipb_mel keeps: a clip of about 10 minutes */
+/* device bytes hipb_mel keeps at most: a clip of about 9 minutes */
 #define CT_MEL_WS_MAX ((size_t)64 << 20)
+
+/* A buffer of at least need bytes for one call: the kept one if it is free and
+ * large enough, else a new one, of a power of two so that ever longer clips
+ * allocate a few times and not on every call. */
+static char *mel_ws_take(HipbEngine *e, size_t need, size_t *bytes) {
+    char *ws = NULL;
+    pthread_mutex_lock(&e->mel_mu);
+    if (e->mel_ws_bytes >= need) {
+        ws = e->mel_ws;
+        *bytes = e->mel_ws_bytes;
+        e->mel_ws = NULL;
+        e->mel_ws_bytes = 0;
+    }
+    pthread_mutex_unlock(&e->mel_mu);
+    if (ws) return ws;
+    *bytes = need;
+    if (need <= CT_MEL_WS_MAX)
+        for (*bytes = (size_t)1 << 20; *bytes < need; *bytes *= 2) {}
+    return dmalloc(*bytes);
+}
+
+/* Gives it back once the call's work is done: the larger one is kept. */
+static void mel_ws_give(HipbEngine *e, char *ws, size_t bytes) {
+    if (bytes <= CT_MEL_WS_MAX) {
+        pthread_mutex_lock(&e->mel_mu);
+        if (bytes > e->mel_ws_bytes) {
+            char *old = e->mel_ws;
+            e->mel_ws = ws;
+            e->mel_ws_bytes = bytes;
+            ws = old;
+        }
+        pthread_mutex_unlock(&e->mel_mu);
+    }
+    if (ws) ECHK(hipFree(ws));
+}
 
 void hipb_mel(HipbEngine *e, const float *pcm, int n_samples, float *mel_out) {
     if (n_samples < HOP_LEN) CT_FATAL("hipb_mel: clip shorter than one hop (160 samples)");
     const int T = 1 + n_samples / HOP_LEN;
-    /* one allocation: clip, frame table, spectrogram, samples */
+    /* one buffer: clip, frame table, spectrogram, samples */
     const size_t o_fc = 256, o_mel = o_fc + ((size_t)T * sizeof(int) + 255) / 256 * 256;
     const size_t o_pcm = o_mel + (size_t)N_MELS * T * 4, need = o_pcm + (size_t)n_samples * 4;
-    pthread_mutex_lock(&e->mel_mu);
-    char *ws = e->mel_ws;
-    if (need > e->mel_ws_bytes) {
-        ws = dmalloc(need);
-        if (need <= CT_MEL_WS_MAX) {
-            if (e->mel_ws) ECHK(hipFree(e->mel_ws));
-            e->mel_ws = ws;
-            e->mel_ws_bytes = need;
-        }
-    }
+    size_t bytes;
+    char *ws = mel_ws_take(e, need, &bytes);
     float *dp = (float *)(ws + o_pcm), *dm = (float *)(ws + o_mel);
     CtMelClip *dc = (CtMelClip *)ws;
     int *fc = (int *)(ws + o_fc);
@@ -1872,6 +1899,5 @@ void hipb_mel(HipbEngine *e, const float *pcm, int n_samples, float *mel_out) {
     ctk_mel(dm, dc, 1, fc, T, &e->mel_tab, e->s);
     ECHK(hipMemcpyAsync(mel_out, dm, (size_t)N_MELS * T * 4, hipMemcpyDeviceToHost, e->s));
     ECHK(hipStreamSynchronize(e->s));
-    if (ws != e->mel_ws) ECHK(hipFree(ws));
-    pthread_mutex_unlock(&e->mel_mu);
+    mel_ws_give(e, ws, bytes);
 }

@@ -108,7 +108,9 @@ int  hipb_chunk_bounds(const float *pcm, int n_samples, float silence_db, float 
  * returns). */
 int  hipb_submit_pcm_device(HipbEngine *e, const float *dev_pcm, int n_samples, const int *prompt,
                             int n_prompt, int limit, int flags);
-/* Log-mel of one clip on the GPU, synchronously (N_MELS x (1 + n/160)). */
+/* Log-mel of one clip on the GPU, synchronously (N_MELS x (1 + n/160)).
+ * Threads may call it at the same time.  The engine keeps one device buffer
+ * of at most 64 MB for its next call. */
 void hipb_mel(HipbEngine *e, const float *pcm, int n_samples, float *mel_out);
 /* Drops every request and frees all slots (caches and weights stay). */
 void hipb_reset(HipbEngine *e);

@@ -8,6 +8,7 @@ test_gpu_engine.py derives for it (twiddle recurrence against exact twiddles).
 """
 import ctypes as C
 import hashlib
+import threading
 
 import numpy as np
 import pytest
@@ -58,6 +59,59 @@ def test_mel_bits(hip, kernel_model):
             x = (np.random.default_rng(n).integers(-8192, 8193, n) / np.float32(32768)).astype(np.float32)
             print(f"case: mel bits n={n}", flush=True)
             assert hashlib.sha256(eng.mel(x).tobytes()).hexdigest()[:16] == want, n
+    finally:
+        eng.close()
+
+
+def test_mel_kept_buffer(hip, kernel_model):
+    """Ever longer clips reuse one buffer of at most 64 MB: the device's free
+    memory stays where the first of them left it, also past a clip too long for
+    a kept buffer (10 M samples: 73 MB)."""
+    rt = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def left():
+        assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    hip.backend_weights_upload_blob(kernel_model.data_ptr, kernel_model.data_bytes)
+    eng = cb.Engine(kernel_model, slots=1, max_requests=2, max_frames=40, kv_bf16=True)
+    try:
+        before, after = left(), []
+        for n in (4_800_000, 5_600_000, 6_400_000, 8_000_000, 10_000_000, 160):
+            print(f"case: mel kept buffer n={n}", flush=True)
+            eng.mel(np.zeros(n, np.float32))
+            after.append(left())
+        assert before - after[0] <= 66 << 20            # the allocator's granule is 2 MB
+        assert after == after[:1] * len(after)
+    finally:
+        eng.close()
+
+
+def test_mel_threads(hip, kernel_model):
+    """Four threads on one engine, clips of all sizes at once: each gets its
+    clip's bits."""
+    hip.backend_weights_upload_blob(kernel_model.data_ptr, kernel_model.data_bytes)
+    eng = cb.Engine(kernel_model, slots=1, max_requests=2, max_frames=40, kv_bf16=True)
+    sizes = [160, 655520, 16000, 320000, 1000, 163000]
+    clips = {n: (np.random.default_rng(n).integers(-8192, 8193, n) / np.float32(32768)).astype(np.float32) for n in sizes}
+    wrong = []
+
+    def work(k):
+        for i in range(18):
+            n = sizes[(i * (k + 1) + k) % len(sizes)]
+            got = hashlib.sha256(eng.mel(clips[n]).tobytes()).hexdigest()[:16]
+            if got != MEL_BITS[n]:
+                wrong.append((k, i, n))
+
+    try:
+        print("case: mel on four threads", flush=True)
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong
     finally:
         eng.close()
 
