@@ -9,6 +9,7 @@
 #include "../../include/model_types.h"
 #include <stdio.h>
 #include <stdlib.h>
+#include <type_traits>
 
 namespace {
 
@@ -375,10 +376,12 @@ __device__ __forceinline__ int packed_owner(const int *off, int n, int tau) {
 // shares with this one and a mel bin: 6 conv values and 4 bins an output,
 // where computing every tap's conv value takes 9 values and 81 LDS reads.  It
 // is bound by its multiply-adds (63 an output and channel).  Every value is
-// summed in the order of sub_conv0 then sub_dwconv (taps in order; a tap
-// outside adds zero), so with finite weights the result is bit-identical to
-// running the two stages (backends/cpu/backend.c:201-221).  The output is
-// written split hi/lo for the pointwise GEMM that reads it.
+// summed in the order of sub_conv0 then sub_dwconv (taps in order, those
+// outside skipped, whatever their weights are), so the result is bit-identical
+// to running the two stages (backends/cpu/backend.c:201-221).  The skips are
+// tests of whole-workgroup conditions, made only in the outputs that have a
+// tap outside: a clip's first and last rows and each row's first column.  The
+// output is written split hi/lo for the pointwise GEMM that reads it.
 // 24 clips (4134 rows) 199 -> 77 us; one clip of 10 s (251 rows) 11.6, where
 // the two stages took 60.
 constexpr int SUB_SEG = 8;                        // output columns of a workgroup
@@ -416,37 +419,45 @@ __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_
         b.f[4] = y.x; b.f[5] = y.y; b.f[6] = y.z; b.f[7] = y.w;
         return b;
     };
-    // the three conv values of one column (rows 2*oh - 1 .. 2*oh + 1) from its
-    // three bins; zero in rows outside the conv output
+    // The three conv values of one column (rows 2*oh - 1 .. 2*oh + 1) from its
+    // three bins.  edge: frames may lie outside the clip, and bin x0 where not in0.
     struct Col { float v[3]; };
-    auto conv = [&](const Bin &x0, const Bin &x1, const Bin &x2) {
+    auto conv = [&](auto edge, const Bin &x0, const Bin &x1, const Bin &x2, bool in0) {
+        constexpr bool E = decltype(edge)::value;
         Col q;
 #pragma unroll
         for (int kh2 = 0; kh2 < 3; kh2++) {
-            const int ih1 = 2 * oh - 1 + kh2;
             float x = bias0;
 #pragma unroll
             for (int kh = 0; kh < 3; kh++) {
-                x += x0.f[2 * kh2 + kh] * k0[kh * 3];
-                x += x1.f[2 * kh2 + kh] * k0[kh * 3 + 1];
-                x += x2.f[2 * kh2 + kh] * k0[kh * 3 + 2];
+                const int f = 2 * kh2 + kh;
+                if (E && (f0 + f < 0 || f0 + f >= T_mel)) continue;
+                if (!E || in0) x += x0.f[f] * k0[kh * 3];
+                x += x1.f[f] * k0[kh * 3 + 1];
+                x += x2.f[f] * k0[kh * 3 + 2];
             }
-            q.v[kh2] = ih1 >= 0 && ih1 < H1 && x > 0.0f ? x : 0.0f;
+            q.v[kh2] = x > 0.0f ? x : 0.0f;
         }
         return q;
     };
+    using Edge = std::true_type;
+    using Inner = std::false_type;
+    const bool edge_rows = f0 < 0 || f0 + 7 > T_mel;      // the row has taps outside the clip
     Bin last = bin(2);                            // bin 4*ow - 1
-    Col left = conv(bin(0), bin(1), last);        // conv column 2*ow - 1
-    if (ow0 == 0) left.v[0] = left.v[1] = left.v[2] = 0.0f;
+    // conv column 2*ow - 1 (of column -1 nothing is used)
+    Col left = edge_rows ? conv(Edge(), bin(0), bin(1), last, true) : conv(Inner(), bin(0), bin(1), last, true);
     const long orow = ((long)tau * 32 + ow0) * SUB_CH + c;
-#pragma unroll 2
-    for (int j = 0; j < SUB_SEG; j++) {
+    auto output = [&](auto edge, int j) {
+        constexpr bool E = decltype(edge)::value;
+        const bool in0 = ow0 + j > 0;             // column 0 has no column and no bin to its left
         const Bin x1 = bin(4 * j + 3), x2 = bin(4 * j + 4), x3 = bin(4 * j + 5), x4 = bin(4 * j + 6);
-        const Col mid = conv(last, x1, x2), right = conv(x2, x3, x4);
+        const Col mid = conv(edge, last, x1, x2, in0), right = conv(edge, x2, x3, x4, true);
         float acc = biasd;
 #pragma unroll
         for (int kh2 = 0; kh2 < 3; kh2++) {
-            acc += left.v[kh2] * kd[kh2 * 3];
+            const int ih1 = 2 * oh - 1 + kh2;
+            if (E && (ih1 < 0 || ih1 >= H1)) continue;
+            if (!E || in0) acc += left.v[kh2] * kd[kh2 * 3];
             acc += mid.v[kh2] * kd[kh2 * 3 + 1];
             acc += right.v[kh2] * kd[kh2 * 3 + 2];
         }
@@ -456,7 +467,11 @@ __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_
         out_lo[orow + (long)j * SUB_CH] = ll;
         left = right;
         last = x4;
-    }
+    };
+    int j = 0;
+    for (const int je = edge_rows ? SUB_SEG : ow0 == 0 ? 1 : 0; j < je; j++) output(Edge(), j);
+#pragma unroll 2
+    for (; j < SUB_SEG; j++) output(Inner(), j);
 }
 
 // sub_dwconv_kernel over several requests, written split hi/lo for the
@@ -465,7 +480,8 @@ __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_
 // [sum (H+1)/2][(Wd+1)/2][256] (without tables, one request of H_arg rows).
 // Workgroup = one output row and SUB_SEG of its columns, thread = channel: the
 // 2*SUB_SEG + 1 input columns of the three rows all in flight at once, each
-// read once; each sum is the scalar form's order (taps outside add zero).
+// read once; each sum is the scalar form's (taps in order, those outside
+// skipped: whole-workgroup conditions).
 // 24 clips (2071 rows) 91 -> 36 us.
 __global__ __launch_bounds__(256) void sub_dw_split_packed_kernel(uint16_t *out_hi, uint16_t *out_lo,
                                                                   const float *in, const int *oin,
@@ -496,9 +512,16 @@ __global__ __launch_bounds__(256) void sub_dw_split_packed_kernel(uint16_t *out_
         if (ow0 + j >= Wo) break;
         float s = bias;
 #pragma unroll
-        for (int kh = 0; kh < 3; kh++)
+        for (int kh = 0; kh < 3; kh++) {
+            const int ih = oh * 2 - 1 + kh;
+            if (ih < 0 || ih >= H) continue;
 #pragma unroll
-            for (int kw = 0; kw < 3; kw++) s += v[kh][2 * j + kw] * k[kh * 3 + kw];
+            for (int kw = 0; kw < 3; kw++) {
+                const int iw = 2 * (ow0 + j) - 1 + kw;    // < 0 at kw 0, >= Wd at kw 2 alone
+                if ((kw == 0 && iw < 0) || (kw == 2 && iw >= Wd)) continue;
+                s += v[kh][2 * j + kw] * k[kh * 3 + kw];
+            }
+        }
         uint16_t hh, ll;
         split_bf16(s, hh, ll);
         const long o = ((long)tau * Wo + ow0 + j) * SUB_CH + c;
