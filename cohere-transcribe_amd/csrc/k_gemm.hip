@@ -183,10 +183,8 @@ __device__ __forceinline__ void store_out8(const CtGemm &g, int m, int col, floa
 // 48 rows: 1024 x 1024 9.2 -> 5.4, 4096 x 1024 12 -> 8.8, 1024 x 4096
 // 29 -> 13.8, 16384 x 1024 24.6 -> 21.
 // ---------------------------------------------------------------------------
-#ifndef CT_DEC_SPLIT
-#define CT_DEC_SPLIT 8
-#endif
-constexpr int DSPLIT = CT_DEC_SPLIT;
+constexpr int DSPLIT = 8;
+constexpr int DEC_K = 1024;      // every decoder-class K is a multiple
 
 // split_bf16 of eight values, two per conversion instruction
 __device__ __forceinline__ void split8(float4 x0, float4 x1, bf16x8 &hi, bf16x8 &lo) {
@@ -207,6 +205,8 @@ __device__ __forceinline__ void split8(float4 x0, float4 x1, bf16x8 &hi, bf16x8 
 
 template <int RB, int CB, int KP>
 __global__ __launch_bounds__(64 * DSPLIT) void gemm_dec_kernel(CtGemm g) {
+    // a wave's K range is whole groups: no load leaves its range or its row
+    static_assert(DEC_K % (DSPLIT * 32 * KP) == 0, "K range of a wave in whole groups of KP K-steps");
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = lane & 15, kg = lane >> 4;
     const int c0 = blockIdx.x * 16 * CB;
@@ -1995,7 +1995,7 @@ void dispatch(const CtGemm &g, hipStream_t s) {
 // Shapes of the decoder's weights: K = DEC_D, or the FFN down projection
 // (K = DEC_FF, N = DEC_D).  They always take the split-K kernel.
 static bool decoder_class(const CtGemm *g) {
-    return g->epi != CT_EPI_GLU && (g->K == 1024 || (g->K == 4096 && g->N == 1024));
+    return g->epi != CT_EPI_GLU && (g->K == DEC_K || (g->K == 4 * DEC_K && g->N == 1024));
 }
 
 // The 16-byte epilogue needs 8-column groups that stay inside one segment
