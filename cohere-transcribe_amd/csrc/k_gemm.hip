@@ -1526,30 +1526,36 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
     };
     const int wr = wv / C::WC, wc = wv % C::WC;
     // bias and the residual rows first (at clamped indices, used after the
-    // loop): their latency passes under the K loop
+    // loop): their latency passes under the K loop.  A tile of 16 blocks a wave
+    // has no registers for that and reads a column block's rows when it stores it.
+    constexpr bool PRE = RB * CB < 16;
     uint16_t bia[CB];
-    float yres[RB][CO][4];
+    float yres[RB][PRE ? CO : 1][4];
     const bool fm = !GLU && g.nseg == 0 && !g.row_len && g.epi == CT_EPI_FMADD;
     const uint16_t *bp = g.bias ? g.bias : g.W;
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) bia[cb] = bp[min(wcol((wc * CB + cb) * 16 + r), nlim - 1)];
-    if (fm) {
+    auto residual = [&](int cb) {
 #pragma unroll
         for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-            for (int cb = 0; cb < CO; cb++)
+            for (int j = 0; j < 4; j++) {
+                const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j, col = c0 + (wc * CO + cb) * 16 + r;
+                yres[rb][PRE ? cb : 0][j] = g.Y[(long)min(m, g.M - 1) * g.ldy + min(col, g.N - 1)];
+            }
+    };
+    if constexpr (PRE) {
+        if (fm) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j, col = c0 + (wc * CO + cb) * 16 + r;
-                    yres[rb][cb][j] = g.Y[(long)min(m, g.M - 1) * g.ldy + min(col, g.N - 1)];
-                }
-    } else {
+            for (int cb = 0; cb < CO; cb++) residual(cb);
+        } else {
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++)
+            for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-            for (int cb = 0; cb < CO; cb++)
+                for (int cb = 0; cb < CO; cb++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) yres[rb][cb][j] = 0.0f;
+                    for (int j = 0; j < 4; j++) yres[rb][cb][j] = 0.0f;
+        }
     }
     f32x4 acc[RB][CB];
 #pragma unroll
@@ -1706,6 +1712,7 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
             const int col = c0 + (wc * CO + cb) * 16 + r;
             if (col >= g.N) continue;
             const float bc = g.bias ? bf2f(bia[cb]) : 0.0f;
+            if (!PRE && fm) residual(cb);
             const long o0 = (long)mb * ld + (inseg ? col - si * g.seg_w : col);
 #pragma unroll
             for (int rb = 0; rb < RB; rb++) {
@@ -1714,7 +1721,7 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
                 for (int j = 0; j < 4; j++) v[j] = acc[rb][cb][j] + bc;
                 if (fm) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) v[j] = yres[rb][cb][j] + g.scale * v[j];
+                    for (int j = 0; j < 4; j++) v[j] = yres[rb][PRE ? cb : 0][j] + g.scale * v[j];
                 } else if (act == CT_EPI_SILU) {
 #pragma unroll
                     for (int j = 0; j < 4; j++) v[j] = v[j] * sigmoid_hw(v[j]);
@@ -1755,8 +1762,8 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
                 if (GLU) {
                     const float gt = acc[rb][cb + (GLU ? CO : 0)][j] + bg;
                     g.Y[(long)m * g.ldy + col] = s * sigmoid_hw(gt);
-                } else if (fm) {
-                    g.Y[(long)m * g.ldy + col] = yres[rb][cb][j] + g.scale * s;
+                } else if (PRE && fm) {
+                    g.Y[(long)m * g.ldy + col] = yres[rb][PRE ? cb : 0][j] + g.scale * s;
                 } else {
                     store_out(g, m, col, s);
                 }

@@ -3,6 +3,7 @@ needed: nothing here launches work)."""
 import ctypes as C
 import os
 import re
+import struct
 import subprocess
 
 import pytest
@@ -190,3 +191,35 @@ def test_reference_transcribe_links_against_hip_backend():
     assert os.path.realpath(line.split("=>")[1].split()[0]) == os.path.realpath(cb.HIP_LIB)
     r = subprocess.run([TRANSCRIBE_HIP], capture_output=True, text=True, timeout=60)
     assert r.returncode == 1 and "Usage:" in r.stderr
+
+
+def code_objects(path):
+    """The gfx950 code objects bundled in a library built by this repository."""
+    blob = open(path, "rb").read()
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at = blob.find(magic)
+    while at >= 0:
+        n, = struct.unpack_from("<Q", blob, at + 24)
+        p = at + 32
+        for _ in range(n):
+            off, size, length = struct.unpack_from("<QQQ", blob, p)
+            if b"gfx950" in blob[p + 24:p + 24 + length]:
+                yield blob[at + off:at + off + size]
+            p += 24 + length
+        at = blob.find(magic, at + 1)
+
+
+def test_no_kernel_spills(tmp_path):
+    """Every kernel's registers fit: no spills, no scratch memory."""
+    kernels = 0
+    for i, code in enumerate(code_objects(cb.HIP_LIB)):
+        obj = tmp_path / f"{i}.o"
+        obj.write_bytes(code)
+        notes = subprocess.run(["/opt/rocm/llvm/bin/llvm-readelf", "--notes", str(obj)], check=True,
+                               capture_output=True, text=True).stdout
+        for k in re.split(r"\n\s+- \.agpr_count", notes)[1:]:
+            name, spilled, scratch = (re.search(rf"\.{f}:\s+(\S+)", k).group(1)
+                                      for f in ("name", "vgpr_spill_count", "private_segment_fixed_size"))
+            kernels += 1
+            assert (spilled, scratch) == ("0", "0"), name
+    assert kernels > 100
