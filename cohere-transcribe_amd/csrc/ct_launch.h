@@ -74,6 +74,10 @@ void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s);
  * 48128 (hi + lo only), 96128, 128128; 0: the cost model);
  * sizeof(CtGemm) for the tests' struct mirror. */
 void ctk_gemm_force_tile(int rows);
+/* The few-row tile (rows * 1000 + columns) that ctk_gemm (n 1) or
+ * ctk_gemm_group takes for these products in one launch; 0: another kernel,
+ * or for a group single launches.  Host code, launches nothing. */
+int  ctk_gemm_tile(const CtGemm *g, int n);
 int  ctk_gemm_sizeof(void);
 
 /* ---------------- decode GEMM on fragment-ordered activations ----------------

@@ -1829,12 +1829,31 @@ constexpr RowsTile ROWS_TILES[] = {
     {16, 32, true, {2.1f, 1.85f, 1.05f}, {1.6f, 1.6f, 1.6f}},
     {32, 32, false, {3.1f, 1.9f, 1.1f}, {1.6f, 1.6f, 1.6f}},
     {32, 64, true, {4.5f, 3.1f, 2.3f}, {1.6f, 1.6f, 1.6f}},
-    {64, 128, true, {13.f, 7.8f, 5.1f}, {5.5f, 6.0f, 6.0f}},
+    {64, 128, true, {10.6f, 7.8f, 5.2f}, {5.2f, 6.0f, 5.4f}},
     {48, 128, true, {0.f, 6.4f, 0.f}, {0.f, 7.7f, 0.f}},
-    {96, 128, true, {0.f, 11.3f, 7.8f}, {0.f, 7.7f, 6.0f}},
-    {128, 128, true, {0.f, 14.2f, 9.5f}, {0.f, 10.5f, 6.0f}},
+    {96, 128, true, {0.f, 11.3f, 7.5f}, {0.f, 7.7f, 6.0f}},
+    {128, 128, true, {0.f, 14.2f, 8.0f}, {0.f, 10.5f, 10.5f}},
 };
 constexpr int N_ROWS_TILES = sizeof ROWS_TILES / sizeof ROWS_TILES[0];
+
+// Estimated us of w workgroups of tile t per CU, k = K / 1000.  Tiles of one
+// workgroup a CU run in rounds.  Of the hi form of 64 x 128 two share a CU, and
+// the second round's fixed part passes under the first (5120 columns, K = 1280:
+// 12.5 us for one round, 19 for two, where 128 x 128 takes 22 for its one).
+// Further rounds are charged it in full: alone they gain as well (26 and 35 us
+// for three and four), but not in an engine, whose weights come from HBM (7
+// clips of 10 s with three rounds 15.50 ms, with the many-row kernel 15.39).
+// The fp32 form of 32 x 64 past one workgroup a CU is such a pair at any number
+// (2 to 6 rounds: 15, 22, 27, 33, 39 us).  The other small tiles: two share a
+// CU at 1.55 times the cost each.
+static double rows_us(const RowsTile &t, int am, double w, double k) {
+    const double rounds = ceil(w);
+    if (t.tm == 64 && am == A_HI) return rounds * k * t.us[am] + fmax(1, rounds - 1) * t.fix[am];
+    if (t.tm >= 48) return rounds * (k * t.us[am] + t.fix[am]);
+    if (w <= 1) return k * t.us[am] + t.fix[am];
+    if (t.tm == 32 && t.tn == 64 && am == A_F32) return 4.4 * (rounds * k + 1);
+    return w * (1.55 * k * t.us[am] + t.fix[am]);
+}
 
 // grp: the n products of a group launch (g the first of them)
 template <int AM>
@@ -2025,9 +2044,11 @@ static int vector_epilogue_ok(const CtGemm *g) {
     return 1;
 }
 
-// Tile choice of the pre-split kernels, for tests: 0 follows the tile-count
-// model below; 128 or 256 takes that tile wherever it applies (the two give
-// the same bits: the same per-element MFMA sequence).
+// Tile choice, for tests: 0 follows the cost models below; 128 or 256 takes the
+// many-row kernels, of pre-split input with that tile wherever it applies;
+// rows * 1000 + columns takes that few-row tile wherever it has a form
+// (ctk_gemm_tile tells), else the many-row kernels.  All give the same bits:
+// the same per-element MFMA sequence.
 static int g_force_tile = 0;
 extern "C" void ctk_gemm_force_tile(int rows) { g_force_tile = rows; }
 extern "C" int ctk_gemm_sizeof(void) { return (int)sizeof(CtGemm); }
@@ -2055,13 +2076,16 @@ static int prefer_256(int M, int n_nt) {
 
 // Index of the few-row tile to run n products of one K in one launch (all but
 // the first: no GLU), or -1 for the many-row kernels: the lowest
-// estimate of time, from rates measured on the encoder's shapes at 3 to 13056
-// rows (ROWS_TILES; a many-row tile of 128 x 256 takes 21 us per 1000 of K and
-// 8.6 us more, hi + lo).  w: workgroups per CU.  Two small workgroups share a
-// CU at 1.55 times the cost each; the larger tiles run in rounds.  Where the
-// line falls (us, few-row against many-row): 1280 x 5120 hi + lo, 1500 rows
-// 50 against 115, 2700 rows 86 against 118; 3840 x 1280, 1008 rows 30 against
-// 38, 1300 rows 40 against 39.
+// estimate of time, from rates measured on the encoder's shapes at 13 to 3600
+// rows (rows_us; a many-row tile of 128 x 256 takes 21 us per 1000 of K and
+// 8.6 us more, hi + lo; profiles/rows_gemm_sweep.json holds every tile's time
+// at every shape, and the choice is within 15% and 0.5 us of the fastest at
+// all 256).  w: workgroups per CU.  Where the line falls (us, few-row against
+// many-row): 1280 x 5120 hi + lo, 1500 rows 50 against 115, 2700 rows 86
+// against 118; 3840 x 1280, 1008 rows 30 against 38, 1300 rows 40 against 39.
+// As tiles run in rounds, the choice can turn back as rows grow: fp32
+// 1280 x 1280 takes 64 x 128 up to 1600 rows (one round), 32 x 64 to 2048
+// (1800 rows: five rounds 34 us, two of 64 x 128 37), and 64 x 128 again.
 static int rows_tile(const CtGemm *g, int am, int n = 1) {
     const bool glu = g->epi == CT_EPI_GLU;
     auto wgs = [&](int tm, int tc) {
@@ -2080,8 +2104,7 @@ static int rows_tile(const CtGemm *g, int am, int n = 1) {
         const RowsTile &t = ROWS_TILES[i];
         if ((glu && !t.glu) || t.us[am] == 0) continue;
         const double w = wgs(t.tm, glu ? t.tn / 2 : t.tn);
-        const double us = t.tm >= 48 ? ceil(w) * (k * t.us[am] + t.fix[am])
-                                     : k * t.us[am] * (w <= 1 ? 1 : 1.55 * w) + t.fix[am] * (w <= 1 ? 1 : w);
+        const double us = rows_us(t, am, w, k);
         if (g_force_tile ? g_force_tile == t.tm * 1000 + t.tn : best < 0 || us < bt) { best = i; bt = us; }
     }
     if (g_force_tile) return best;
@@ -2092,6 +2115,29 @@ static int rows_tile(const CtGemm *g, int am, int n = 1) {
     double many = ceil(w) * one;
     if (g->M >= CT_SPLIT256_MIN_M && 1.74 * ceil(w2) * one < many) many = 1.74 * ceil(w2) * one;
     return bt < many ? best : -1;
+}
+
+// fp32 rows and weight rows that can be read in 16-byte pieces
+static bool vec_rows(const CtGemm *g) {
+    return (g->K % 8 == 0) && (g->lda % 4 == 0) && (((uintptr_t)g->A & 15) == 0) && (((uintptr_t)g->W & 15) == 0);
+}
+
+// Few-row tile of a product by itself, or of n as one launch; -1: none.
+static int single_tile(const CtGemm *g) {
+    if (g->Ahi) return rows_tile(g, g->Alo ? A_HILO : A_HI);
+    return vec_rows(g) && !decoder_class(g) ? rows_tile(g, A_F32) : -1;
+}
+static int group_tile(const CtGemm *g, int n) {
+    if (n < 2 || n > CT_GEMM_GROUP) return -1;
+    for (int i = 0; i < n; i++)
+        if (g[i].M <= 0 || g[i].N <= 0 || g[i].Ahi || g[i].epi == CT_EPI_GLU || g[i].K != g->K ||
+            single_tile(&g[i]) < 0)               // its own address spans too
+            return -1;
+    return rows_tile(g, A_F32, n);
+}
+extern "C" int ctk_gemm_tile(const CtGemm *g, int n) {
+    const int rt = n > 1 ? group_tile(g, n) : single_tile(g);
+    return rt < 0 ? 0 : ROWS_TILES[rt].tm * 1000 + ROWS_TILES[rt].tn;
 }
 
 extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
@@ -2108,7 +2154,7 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
             exit(1);
         }
         const bool glu = g->epi == CT_EPI_GLU;
-        const int rt = rows_tile(g, g->Alo ? A_HILO : A_HI);
+        const int rt = single_tile(g);
         if (rt >= 0) return g->Alo ? launch_rows<A_HILO>(rt, *g, s) : launch_rows<A_HI>(rt, *g, s);
         const int n_mt = (g->M + SBM - 1) / SBM;
         const int n_nt = glu ? (g->glu_half + SBN / 2 - 1) / (SBN / 2) : (g->N + SBN - 1) / SBN;
@@ -2131,8 +2177,7 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
         else hipLaunchKernelGGL((gemm_split_kernel<false, false>), dim3(per * 8), dim3(512), 0, s, *g, n_mt, n_nt, vepi);
         return;
     }
-    const bool vec = (g->K % 8 == 0) && (g->lda % 4 == 0) &&
-                     (((uintptr_t)g->A & 15) == 0) && (((uintptr_t)g->W & 15) == 0);
+    const bool vec = vec_rows(g);
     const bool glu = g->epi == CT_EPI_GLU;
     if (vec && decoder_class(g)) {
         // The smallest tile whose workgroups all run at once: below that the
@@ -2148,7 +2193,7 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
         else launch_dec<2, 4, 2>(*g, s);
         return;
     }
-    const int rt = vec ? rows_tile(g, A_F32) : -1;
+    const int rt = single_tile(g);
     if (rt >= 0) return launch_rows<A_F32>(rt, *g, s);
     if (vec && g->K % BK == 0 && g->M > 64) {
         // same per-element MFMA sequence as the small-M kernels: bit-identical rows
@@ -2171,12 +2216,7 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
 // 2T - 1) as one launch: 7.8 us at T = 13 (6.6 each alone), 16 at 101 (8 and
 // 11), 41 at 376 (11 and 22).
 extern "C" void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s) {
-    bool one = n > 1 && n <= CT_GEMM_GROUP;
-    for (int i = 0; one && i < n; i++)
-        one = g[i].M > 0 && g[i].N > 0 && !g[i].Ahi && g[i].epi != CT_EPI_GLU && g[i].K == g->K && g[i].lda % 4 == 0 &&
-              ((uintptr_t)g[i].A & 15) == 0 && ((uintptr_t)g[i].W & 15) == 0 && !decoder_class(&g[i]) &&
-              rows_tile(&g[i], A_F32) >= 0;       // its own address spans too
-    const int rt = one ? rows_tile(g, A_F32, n) : -1;
+    const int rt = group_tile(g, n);
     if (rt < 0) {
         for (int i = 0; i < n; i++) ctk_gemm(&g[i], s);
         return;
