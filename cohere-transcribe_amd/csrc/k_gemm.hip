@@ -2094,9 +2094,10 @@ static int rows_tile(const CtGemm *g, int am, int n = 1) {
             t += (double)((g[i].M + tm - 1) / tm) * (((glu ? g->glu_half : g[i].N) + tc - 1) / tc);
         return t / cu_count();
     };
-    // every DMA address is a base and a 32-bit offset within the tile's rows
+    // every DMA address is a base and a 32-bit unsigned offset within the tile's
+    // rows; an empty sum (K = 0) has no stage to fetch and no weights to read
     const long wspan = (long)(glu ? g->glu_half + 256 : 256) * g->K * 2, aspan = 128L * g->lda * 4;
-    if (g->K % 128 || wspan >= 1L << 31 || aspan >= 1L << 31) return -1;
+    if (g->K <= 0 || g->K % 128 || g->lda < 0 || wspan >= 1L << 31 || aspan >= 1L << 31) return -1;
     const double k = g->K / 1000.0;
     int best = -1;
     double bt = 0;

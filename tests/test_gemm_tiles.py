@@ -49,3 +49,18 @@ def test_choice_is_near_the_fastest(lib):
         if mine > 1.15 * min(us.values()) + 0.5:
             slow.append((M, N, K, act, epi, tile, mine, us))
     assert not slow
+
+
+@pytest.mark.parametrize("act", ["fp32", "hilo", "hi"])
+def test_what_the_few_row_kernel_cannot_take(lib, act):
+    """An empty sum (its clamped loads would read weights that are not there),
+    rows that run backwards or are further apart than 32-bit offsets reach, and
+    a K outside its stages go to the general kernels, alone and in a group."""
+    def tiles(**over):
+        g = gemm(101, 1280, over.pop("K", 1280), act, **over)
+        two = (CtGemm * 2)(g, g)
+        return lib.ctk_gemm_tile(C.byref(g), 1), lib.ctk_gemm_tile(two, 2)
+    alone, grouped = tiles()
+    assert alone and bool(grouped) == (act == "fp32")
+    for over in ({"K": 0, "lda": 1280}, {"K": 1312}, {"lda": -1280}, {"lda": 1 << 22}):
+        assert tiles(**over) == (0, 0), over
