@@ -2054,13 +2054,12 @@ extern "C" void ctk_gemm_force_tile(int rows) { g_force_tile = rows; }
 extern "C" int ctk_gemm_sizeof(void) { return (int)sizeof(CtGemm); }
 
 static int cu_count(void) {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-            cus = 256;
-    }
+    static const int cus = [] {           // set once, whichever thread is first
+        int dev = 0, n = 0;
+        const bool ok = hipGetDevice(&dev) == hipSuccess &&
+                        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
+        return ok && n > 0 ? n : 256;
+    }();
     return cus;
 }
 
@@ -2072,7 +2071,6 @@ static int prefer_256(int M, int n_nt) {
     const double r128 = (double)((t128 + cus - 1) / cus), r256 = (double)((t256 + cus - 1) / cus);
     return r256 * 1.74 < r128;
 }
-
 
 // Index of the few-row tile to run n products of one K in one launch (all but
 // the first: no GLU), or -1 for the many-row kernels: the lowest
