@@ -4,7 +4,8 @@ workgroups, and longer than the rows kept in registers (4096 frames); rows of
 logits of whole float4 and not, with ties, NaN and infinities.
 
 The spectrogram is held to the oracle's within the tolerance that
-test_gpu_engine.py derives for it (twiddle recurrence against exact twiddles).
+test_gpu_engine.py derives for it (twiddle recurrence against exact twiddles),
+and to a restatement in float64.
 """
 import ctypes as C
 import hashlib
@@ -32,6 +33,45 @@ def test_mel_lengths(hip, kernel_model):
             assert got.shape == ref.shape
             assert np.abs(got - ref).max() < 2e-3, n
             assert np.array_equal(got, eng.mel(x))
+    finally:
+        eng.close()
+
+
+def mel64(x):
+    """The log-mel spectrogram in float64 (window and filters included)."""
+    n, T = len(x), 1 + len(x) // 160
+    x = x.astype(np.float64)
+    e = np.concatenate([np.zeros(200), x, np.zeros(200 + 160)])
+    e[1:] -= 0.97 * e[:-1].copy()
+    hann = 0.5 * (1 - np.cos(2 * np.pi * np.arange(400) / 399))
+    spec = np.array([np.abs(np.fft.rfft(e[160 * t:160 * t + 400] * hann, 512)) ** 2 for t in range(T)])
+    def hz(m):
+        return np.where(m < 15, m * 200 / 3, 1000 * np.exp((m - 15) * np.log(6.4) / 27))
+    top = 15 + np.log(8.0) / (np.log(6.4) / 27)
+    p = hz(np.linspace(0, top, 130))
+    f = np.linspace(0, 8000, 257)
+    fb = [np.maximum(0, np.minimum((f - p[i]) / (p[i + 1] - p[i]), (p[i + 2] - f) / (p[i + 2] - p[i + 1]))) * 2 / (p[i + 2] - p[i])
+          for i in range(128)]
+    mel = np.log(np.array(fb) @ spec.T + 2.0 ** -24)
+    d = mel - mel.mean(1, keepdims=True)
+    return d / np.sqrt((d ** 2).sum(1, keepdims=True) / (T - 1) + 1e-5)
+
+
+@pytest.mark.parametrize("n", [3 * 160, 8000, 48000, 327680, 655520])
+def test_mel_float64(hip, kernel_model, n):
+    """Against float64 in the 2-norm.  Nine butterfly stages of three roundings
+    of 2^-24, twice in the power and again its logarithm's absolute error: 27
+    2^-23 = 3.2e-6, and a row's standard deviation here is 0.5 and more; the
+    window and the filters are rounded once (2^-24)."""
+    hip.backend_weights_upload_blob(kernel_model.data_ptr, kernel_model.data_bytes)
+    eng = cb.Engine(kernel_model, slots=1, max_requests=2, max_frames=40, kv_bf16=True)
+    try:
+        x = (np.random.default_rng(n).integers(-8192, 8193, n) / np.float32(32768)).astype(np.float32)
+        print(f"case: mel float64 n={n}", flush=True)
+        got, ref = eng.mel(x).astype(np.float64), mel64(x)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        print(f"  relative error {err:.2e}", flush=True)
+        assert err <= 7e-6
     finally:
         eng.close()
 
