@@ -1535,19 +1535,17 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
     const uint16_t *bp = g.bias ? g.bias : g.W;
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) bia[cb] = bp[min(wcol((wc * CB + cb) * 16 + r), nlim - 1)];
-    auto residual = [&](int cb) {
-#pragma unroll
-        for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j, col = c0 + (wc * CO + cb) * 16 + r;
-                yres[rb][PRE ? cb : 0][j] = g.Y[(long)min(m, g.M - 1) * g.ldy + min(col, g.N - 1)];
-            }
-    };
     if constexpr (PRE) {
         if (fm) {
 #pragma unroll
-            for (int cb = 0; cb < CO; cb++) residual(cb);
+            for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                for (int cb = 0; cb < CO; cb++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const int m = m0 + (wr * RB + rb) * 16 + kg * 4 + j, col = c0 + (wc * CO + cb) * 16 + r;
+                        yres[rb][cb][j] = g.Y[(long)min(m, g.M - 1) * g.ldy + min(col, g.N - 1)];
+                    }
         } else {
 #pragma unroll
             for (int rb = 0; rb < RB; rb++)
@@ -1712,7 +1710,13 @@ __device__ __forceinline__ void rows_body(const CtGemm &g, int t, int n_mt, char
             const int col = c0 + (wc * CO + cb) * 16 + r;
             if (col >= g.N) continue;
             const float bc = g.bias ? bf2f(bia[cb]) : 0.0f;
-            if (!PRE && fm) residual(cb);
+            if (!PRE && fm) {
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        yres[rb][0][j] = g.Y[(long)min(mb + rb * 16 + j, g.M - 1) * g.ldy + col];
+            }
             const long o0 = (long)mb * ld + (inseg ? col - si * g.seg_w : col);
 #pragma unroll
             for (int rb = 0; rb < RB; rb++) {
@@ -1847,10 +1851,10 @@ constexpr int N_ROWS_TILES = sizeof ROWS_TILES / sizeof ROWS_TILES[0];
 // (2 to 6 rounds: 15, 22, 27, 33, 39 us).  The other small tiles: two share a
 // CU at 1.55 times the cost each.
 static double rows_us(const RowsTile &t, int am, double w, double k) {
-    const double rounds = ceil(w);
-    if (t.tm == 64 && am == A_HI) return rounds * k * t.us[am] + fmax(1, rounds - 1) * t.fix[am];
-    if (t.tm >= 48) return rounds * (k * t.us[am] + t.fix[am]);
     if (w <= 1) return k * t.us[am] + t.fix[am];
+    const double rounds = ceil(w);
+    if (t.tm == 64 && am == A_HI) return rounds * k * t.us[am] + (rounds - 1) * t.fix[am];
+    if (t.tm >= 48) return rounds * (k * t.us[am] + t.fix[am]);
     if (t.tm == 32 && t.tn == 64 && am == A_F32) return 4.4 * (rounds * k + 1);
     return w * (1.55 * k * t.us[am] + t.fix[am]);
 }
