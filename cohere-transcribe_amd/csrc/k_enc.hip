@@ -382,7 +382,7 @@ __device__ __forceinline__ int packed_owner(const int *off, int n, int tau) {
 // tests of whole-workgroup conditions, made only in the outputs that have a
 // tap outside: a clip's first and last rows and each row's first column.  The
 // output is written split hi/lo for the pointwise GEMM that reads it.
-// 24 clips (4134 rows) 199 -> 77 us; one clip of 10 s (251 rows) 11.6, where
+// 24 clips (4134 rows) 199 -> 71 us; one clip of 10 s (251 rows) 9.7, where
 // the two stages took 60.
 constexpr int SUB_SEG = 8;                        // output columns of a workgroup
 __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_hi, uint16_t *out_lo,
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(256) void sub_conv0_dw_packed_kernel(uint16_t *out_
 // 2*SUB_SEG + 1 input columns of the three rows all in flight at once, each
 // read once; each sum is the scalar form's (taps in order, those outside
 // skipped: whole-workgroup conditions).
-// 24 clips (2071 rows) 91 -> 36 us.
+// 24 clips (2071 rows) 91 -> 38 us.
 __global__ __launch_bounds__(256) void sub_dw_split_packed_kernel(uint16_t *out_hi, uint16_t *out_lo,
                                                                   const float *in, const int *oin,
                                                                   const int *oout, int n, int H_arg, int Wd,

@@ -1389,7 +1389,9 @@ __global__ __launch_bounds__(512) void gemm_split256_sp_kernel(CtGemm g, int n_m
 // scalar base and a constant lane offset, and, for fp32 activations, split
 // each 16 x 32 fragment into hi and lo once per workgroup, two stages ahead.
 // One barrier per stage.  LDS rows are swizzled for both the DMA (1 KB runs)
-// and the fragment reads.  In the 64- and 96-row tiles waves have both roles.
+// and the fragment reads.  In the 64-row tile and in the 96-row tile of hi + lo
+// planes every wave has both roles, in the 96-row tile of the hi plane half of
+// the MFMA waves fetch as well.
 //
 // Measured (us; before -> now): fp32 activations 13 x 1280 x 1280 15 -> 6.6,
 // 101 x 1280 x 5120 161 -> 21, 376 x 5120 x 1280 49 -> 22; hi + lo planes
@@ -2187,7 +2189,9 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
         // weights and activations a CU reads grow, above it a second round
         // starts.  1024 x 1024 x 48 rows: 16 x 16 5.4 us, 16 x 32 6.5, 32 x 32
         // 8.2; 4096 x 1024 x 64: 32 x 32 8.8, 16 x 16 14; 16384 x 1024 x 48:
-        // 32 x 64 21, 16 x 64 23.
+        // 32 x 64 21, 16 x 64 23.  Past 64 rows (a clip's cross keys and values,
+        // 16 products of T x 1024 x 1024; us, one workgroup per 64 x 16 before):
+        // T = 65 193 -> 98, 160 194 -> 136, 376 315 -> 182, 4000 2120 -> 1310.
         const long nt = (g->N + 15) / 16, mt = (g->M + 15) / 16, cus = cu_count();
         if (nt * mt <= cus) launch_dec<1, 1, 4>(*g, s);
         else if ((nt + 1) / 2 * mt <= cus) launch_dec<1, 2, 4>(*g, s);
@@ -2216,8 +2220,8 @@ extern "C" void ctk_gemm(const CtGemm *g, hipStream_t s) {
 // Products of fp32 activations and one K that do not depend on each other: in
 // one launch where they take a few-row tile together, else one by one.  The
 // four projections of relative-position attention (Q, K, V of T rows, P of
-// 2T - 1) as one launch: 7.8 us at T = 13 (6.6 each alone), 16 at 101 (8 and
-// 11), 41 at 376 (11 and 22).
+// 2T - 1) as one launch: 7.4 us at T = 13 (6.6 each alone), 15 at 101 (8 and
+// 11), 36 at 376 (12 and 20).
 extern "C" void ctk_gemm_group(const CtGemm *g, int n, hipStream_t s) {
     const int rt = group_tile(g, n);
     if (rt < 0) {

@@ -28,7 +28,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // split over the workgroup (WPF 4): one butterfly a lane and a barrier per
 // stage.  Both do the same arithmetic per element.  us, WPF 1 and 4: 51 frames
 // 11.3 and 6.3, 301 11.9 and 6.7, 1019 12.5 and 9.7, 2001 14.2 and 14.4, 3001
-// 18.3 and 18.4, 4096 20.9 and 22.9, 6251 29 and 32; 16503 with WPF 1 63 (89
+// 18.3 and 18.4, 4096 20.9 and 22.9, 6251 29 and 32; 16503 with WPF 1 58 (89
 // with twiddles from memory and two barriers a stage).
 constexpr int MEL_FEW_FRAMES = 2048;
 template <int WPF>
