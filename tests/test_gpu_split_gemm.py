@@ -12,6 +12,7 @@ through libct_hip.so's C entry point.
   float64 product of those values the fp32 sums agree to 1e-5, and an output
   rounded to bf16 lies within one bf16 step of the float64 value.
 * A row's bits do not depend on how many rows the launch has.
+* The few-row tiles give the same bits through the same output modes.
 * GLU (the conv module's first pointwise projection): value column j times
   the sigmoid of gate column j + N/2, both with their bias.
 
@@ -43,6 +44,8 @@ def lib(hip):
     assert C.sizeof(CtGemm) == L.ctk_gemm_sizeof()
     L.ctk_gemm.argtypes = [C.POINTER(CtGemm), C.c_void_p]
     L.ctk_gemm_force_tile.argtypes = [C.c_int]
+    L.ctk_gemm_tile.argtypes = [C.POINTER(CtGemm), C.c_int]
+    L.ctk_gemm_tile.restype = C.c_int
     yield L
     L.ctk_gemm_force_tile(0)
 
@@ -242,3 +245,28 @@ def test_split_gemm_tiles_modes_and_float64(lib, hip, mode, N, K, lo):
         e = np.abs(got - np.maximum(s, 0.0)).max() / scale
         print(f"  relerr {e:.2e}")
         assert e <= 1e-5
+
+
+FEW_ROW = [16016, 16032, 32032, 32064, 64128, 48128, 96128, 128128]
+
+
+@pytest.mark.parametrize("lo", [True, False], ids=["hilo", "single"])
+@pytest.mark.parametrize("mode,N,K", MODES, ids=[m[0] for m in MODES])
+def test_few_row_tiles_in_every_mode(lib, hip, mode, N, K, lo):
+    """The engine's products take few-row tiles up to about 3000 rows, by size:
+    every one with a form for the input gives the many-row kernel's bits."""
+    dev = Dev(hip)
+    case = Case(dev, mode, N, K, lo, seed=N + K + lo)
+    ran = 0
+    for M in (M_PART, M_FULL):
+        want = case.run(lib, M, tile=128)
+        for tile in FEW_ROW:
+            lib.ctk_gemm_force_tile(tile)
+            if lib.ctk_gemm_tile(C.byref(case.gemm(M)), 1) != tile:
+                continue
+            print(f"case: few-row {mode} M={M} N={N} K={K} {'hi+lo' if lo else 'single-pass'} tile {tile}", flush=True)
+            for a, b in zip(want, case.run(lib, M, tile=tile)):
+                assert np.array_equal(a, b), (M, tile)
+            ran += 1
+    # K = 1312 is no whole number of stages; one tile has no single-pass form, two none with GLU
+    assert ran == (0 if K % 128 else 2 * (len(FEW_ROW) - (not lo) - 2 * (mode == "glu")))
